@@ -80,7 +80,7 @@ def draw(rng):
     kind = rng.choice(["ffn", "ffn", "linear", "linear", "decode", "decode", "layer", "layer",
                        "head", "request"])
     if kind == "ffn":
-        return {"kind": kind, "n": _log_int(rng, 1, 2048)}
+        return {"kind": kind, "n": _log_int(rng, 2, 2048)}   # one row: the listed case
     if kind == "linear":
         N, K = rng.choice([(8192, 28672), (28672, 8192), (13824, 2560), (2560, 6912),
                            (6912, 2560), (3840, 2560), (2560, 2560), (5120, 8192)])
@@ -95,7 +95,7 @@ def draw(rng):
         return {"kind": kind, "n": n, "pos0": pos0}
     if kind == "head":
         return {"kind": kind, "top_k": rng.choice([0, 1, 40, 50, 50, _log_int(rng, 2, 2000)]),
-                "temperature": rng.choice([1.0, 0.7, round(rng.uniform(0.5, 1.5), 3)]),
+                "temperature": round(rng.uniform(0.5, 1.5), 3),
                 "penalty": rng.choice([1.0, 1.1])}
     # the f32 cache is the reference's own type (a parity mode: shorter prompts)
     if rng.random() < 0.2:
