@@ -1185,80 +1185,112 @@ __global__ __launch_bounds__(kPrefillThreads) void attn_prefill_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Prefill on f32 MFMA.  v_mfma_f32_16x16x1_4b (K = 1) adds one product to
-// each output element per instruction, D = A*B + C rounded once, which is
-// the fused multiply-add: a chain of them over d (or over positions) is the
-// same sequential fma chain as the shaders' loops, bit for bit, at twice the
-// VALU's fma rate.  Lane l supplies A[block l/16][row l%16] and B[block
-// l/16][col l%16]; element (block b, row i, col j) of D is in lane
-// j + 16(i/4), register 4b + i%4.
+// Prefill on f32 MFMA.  v_mfma_f32_16x16x4 adds its four products to each
+// output element one after the other in order of k, each with one rounding
+// (compared on the device with fmaf chains, subnormals included: 0 of 8192
+// chains of 128 steps differ; the reverse order differs in 82%), so a chain
+// of them over d, or over positions, is the shaders' sequential fma chain bit
+// for bit, four steps per instruction.  Lane l supplies A[row l%16][k l/16] and
+// B[k l/16][col l%16] and holds D[row 4(l/16) + i][col l%16] in register i.
+// One dependent chain issues at 32 cycles per instruction, the MFMA's own
+// rate; a VALU instruction between two of them costs it 8 to 16 cycles, also
+// when other waves wait (measured with chains in registers: no VALU 147
+// TFLOP/s from four waves per SIMD, one convert per MFMA 122, from one wave
+// 130 and 96), so the loops below hold MFMAs, loads and nothing else.
 //
-// The B operands come from copies of the cache laid out for them
-// (attn_kv_tiles_kernel, one pass per call): per KV head
-//   Kt [tile of 64 positions][d/4][64 positions][4 d]           f32
-//   Vt [position/4][128 dims][4 positions]         f16
-// zero past the last position, so a lane's 16-byte load is 4 steps of its
-// operand (K with no conversion), and a wave's load is 1 KB contiguous.
+// The A operands come from f32 copies of the cache laid out for them
+// (attn_kv_tiles_kernel, one pass per call), per KV head and 16 positions:
+//   Kt [8 u][64 lanes][4 f32]: element e of lane l is K[position of row
+//      l%16][d = 16u + 4e + l/16]
+//   Vt [8 dim tiles of 16][64 lanes][4 f32]: element e of lane l is
+//      V[position 4e + l/16][dim l%16 of the tile]
+// zero past the last position; each load is 1 KB contiguous per wave and
+// feeds 4 instructions.
 //
-// One workgroup of 16 waves (four per SIMD: a dependent MFMA chain issues at
-// ~64% of the MFMA rate from one wave per SIMD, ~100% from four) per (16/G
-// consecutive queries, KV head): 16 score rows, row r = query r/G, head r%G;
-// query i attends over its position + 1 positions (causal).  The workgroups
-// of one XCD share the K / V copies of at most two KV heads (mapping below).
-//   scores: wave w takes the 64-position tiles w, w+16, ...: per d one
-//     instruction covers the 16 rows (A = q[r][d], the same in the 4 blocks)
-//     x 64 positions (B = K[tile + l][d]), 128 of them in order of d.
-//     dot * scale goes to the row in LDS.
-//   softmax: wave_softmax_row on row w, in place; positions past the row's
-//     length become exact zeros.
-//   P.V (sh/attention.wgsl:96-104): one chain per output over all of its
-//     row's positions, in order of s, on v_mfma_f32_4x4x1_16b (one fused
-//     step per output per instruction; lane l supplies A[block l/4][row
-//     l%4], B[block l/4][col l%4] and holds D[block l/4][row i][col l%4] in
-//     register i).  Wave w < 4 takes rows 8(w%2) .. +7 as two groups of
-//     four (A = p[row][s], two chains per lane) and dims 64(w/2) .. +63 (B =
-//     V[s][64(w/2) + l], one f16 operand for both groups), so the four
-//     waves load each V element twice, 8 bytes per lane per 4 positions, and
-//     hold kPvAhead 16-position batches of it in flight.  Positions that
-//     every row of a wave covers run in whole batches; the last ones keep
-//     each row's sum past its own length (a select per row).
-// LDS (dynamic): q [16][132] | rows [16][Sw], Sw = the longest row rounded
-// up to 64, plus 4, so that the 16 rows one read touches start in different
-// banks.
+// Score rows sit in LDS with each 16 positions permuted: position 4j + k at
+// slot 4k + j, so that the P.V operand of a lane (k = l/16) for four
+// instructions is one 16-byte read.  Row m of a K tile holds the position of
+// slot m, which makes a lane's four scores one 16-byte write.
+//
+// One workgroup of 8 waves per (R/G consecutive queries, KV head): R score
+// rows, row r = query r/G, head r%G; query i attends over its position + 1
+// positions (causal).  R = 16 while 16 rows fit the LDS (two workgroups per
+// CU up to 1216 positions, so that one's softmax overlaps another's MFMAs),
+// else R = 8: columns 8-15 repeat columns 0-7.  The workgroups of one XCD
+// share the K / V copies of at most two KV heads (mapping below).
+//   scores: wave w takes the 16-position tiles w, w+8, ...: 32 instructions
+//     in order of d, A = K (a tile ahead in registers), B = q (32
+//     registers held throughout); the dots to the rows.
+//   softmax: dot * scale, then softmax_row_slots, one wave per row, in place.
+//   P.V (sh/attention.wgsl:96-104): wave w takes dims 16w .. 16w+15, one chain
+//     per output over all positions in order of s, A = V (kPvAhead batches of
+//     16 positions ahead), B = p (one ahead).  The last groups of four, which
+//     not every row reaches whole, run one position per instruction: the other three k
+//     get +0 * -0, which leaves any sum as it is, and each row keeps its sum
+//     past its own length (a select, so nothing beyond a row touches it).
+// LDS (dynamic): rows [R][Sw], Sw = the longest row rounded up to 64, plus 4,
+// so that the 16 rows one read touches start in different banks; the q rows
+// pass through the same memory first.
+// us per call with the copies, 20 / 5 heads, against the design before (16
+// rows, 16x16x1 and 4x4x1 MFMAs with converts between them; VALU past 2368
+// positions): 2048 queries from position 0 361 -> 245, 1000 from 0 106 -> 68,
+// 512 from 2000 (R = 8) 544 -> 231, 64 from 2400 128 -> 59, 1500 from 2500
+// 2041 -> 875, 16-101 from 0 level (28; launches).  Per workgroup at 2048
+// queries (mean clocks): scores 18.2k of 16.4k MFMA clocks, softmax 7.8k,
+// P.V about 17k, the rest 5.6k: one workgroup fits a CU there, and on one
+// SIMD the softmax's VALU time adds to the MFMA time whatever overlaps.
 // ---------------------------------------------------------------------------
-typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
-constexpr int kPfmWaves = 16;
+constexpr int kPfmWaves = 8;
 constexpr int kPfmThreads = 64 * kPfmWaves;
-constexpr int kPfmQs = kHd + 4;   // q row stride (floats)
-constexpr int kPfmMaxS = 2368;    // longest row whose 16 rows fit the LDS (160 KB)
-constexpr int kTileF4 = 64 * kHd / 4;    // float4 of one 64-position tile of Kt
-constexpr int kVTileU4 = 64 * kHd / 8;   // uint4 of one 64-position tile of Vt
-constexpr int kPvAhead = 3;              // P.V: V batches in flight per wave
+constexpr int kPfmQs = kHd + 4;          // q row stride (floats)
+constexpr int kPfmMaxS16 = 2496;         // longest row whose 16 (8) rows fit the LDS (160 KB)
+constexpr int kPfmMaxS8 = 5056;
+constexpr int kKvTile = 16;              // positions per tile of the copies
+constexpr int kTileF4 = kKvTile * kHd / 4;   // float4 of one tile (of Kt, of Vt)
+constexpr int kPvAhead = 9;              // P.V: V batches in flight per wave
 
 __host__ __device__ inline int pfm_row_stride(int s_max) { return ((s_max + 63) & ~63) + 4; }
-__host__ __device__ inline size_t pfm_smem(int s_max) {
-    return (size_t)16 * (kPfmQs + pfm_row_stride(s_max)) * sizeof(float);
+__host__ __device__ inline size_t pfm_smem(int R, int s_max) {
+    const size_t rows = (size_t)R * pfm_row_stride(s_max), q = (size_t)R * kPfmQs;
+    return ((rows > q ? rows : q) + 16) * sizeof(float);   // P.V reads one batch past a row
 }
 
-__device__ __forceinline__ v16f mfma_f32_k1(float a, float b, const v16f &c) {
-    return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 0, 0, 0);
+// A KV head's copy as a buffer, read at a wave-uniform byte offset plus 16
+// bytes per lane: the address takes no VALU instruction, and nothing outside
+// the head's tiles can be read.
+typedef __amdgpu_buffer_rsrc_t CopyRsrc;
+__device__ __forceinline__ CopyRsrc copy_rsrc(const float4 *copy, int hk, int ntile) {
+    return __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(copy + (size_t)hk * ntile * kTileF4), 0, ntile * kTileF4 * 16, 0x00027000);
+}
+__device__ __forceinline__ float4 copy_load(CopyRsrc r, int lane, int off) {
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, 16 * lane, off, 0));
 }
 
-// Kt and Vt tiles (layouts above) of positions [64t, 64t + 64) of KV head hk
-// from the f16 caches; positions >= S are zeros.  Grid (tiles, Hkv).
+// acc += a * b for one float4 of steps (four instructions)
+__device__ __forceinline__ void mfma_steps4(v4f &acc, const float4 &a, const float4 &b) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, acc, 0, 0, 0);
+}
+
+// Kt and Vt (layouts above) of the 16-position tiles 2t and 2t + 1 of KV head
+// hk from the f16 caches (the copies hold an even number of tiles); positions
+// >= S are zeros.  Grid (pairs of tiles, Hkv).
 __global__ __launch_bounds__(256) void attn_kv_tiles_kernel(const uint16_t *__restrict__ kc,
                                                             const uint16_t *__restrict__ vc,
                                                             int max_seq, int S, int ntile_ws,
                                                             float4 *__restrict__ Kt,
-                                                            uint4 *__restrict__ Vt) {
-    __shared__ uint4 ks[64][17], vs[64][17];   // 64 rows of 16 uint4, padded
+                                                            float4 *__restrict__ Vt) {
+    __shared__ uint4 ks[2 * kKvTile][17], vs[2 * kKvTile][17];   // rows of 16 uint4, padded
     const int t = blockIdx.x, hk = blockIdx.y, tid = threadIdx.x;
     const uint4 *K4 = (const uint4 *)(kc + (size_t)hk * max_seq * kHd);
     const uint4 *V4 = (const uint4 *)(vc + (size_t)hk * max_seq * kHd);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int i = tid + 256 * k, row = i >> 4, c = i & 15, pos = 64 * t + row;
+    for (int k = 0; k < 2; ++k) {
+        const int i = tid + 256 * k, row = i >> 4, c = i & 15, pos = 2 * kKvTile * t + row;
         uint4 kv = make_uint4(0, 0, 0, 0), vv = make_uint4(0, 0, 0, 0);
         if (pos < S) {
             kv = K4[(size_t)pos * 16 + c];
@@ -1268,34 +1300,100 @@ __global__ __launch_bounds__(256) void attn_kv_tiles_kernel(const uint16_t *__re
         vs[row][c] = vv;
     }
     __syncthreads();
-    auto h2f = [](uint32_t h) { return __half2float(__ushort_as_half((uint16_t)h)); };
-    float4 *kt = Kt + ((size_t)hk * ntile_ws + t) * kTileF4;
+    auto h2f = [](uint16_t h) { return __half2float(__ushort_as_half(h)); };
+    float4 *kt = Kt + ((size_t)hk * ntile_ws + 2 * t) * kTileF4;
+    float4 *vt = Vt + ((size_t)hk * ntile_ws + 2 * t) * kTileF4;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {   // kt[c][p]: dims 4c .. 4c+3 of position p
-        const int i = tid + 256 * k, c = i >> 6, pos = i & 63;
-        const uint4 u = ks[pos][c >> 1];
-        const uint32_t lo = (c & 1) ? u.z : u.x, hi = (c & 1) ? u.w : u.y;
-        kt[i] = make_float4(h2f(lo & 0xffff), h2f(lo >> 16), h2f(hi & 0xffff), h2f(hi >> 16));
-    }
-    uint2 *vt = (uint2 *)(Vt + ((size_t)hk * ntile_ws + t) * kVTileU4);
+    for (int k = 0; k < 4; ++k) {
+        const int i = tid + 256 * k, l = i & 63, m = l & 15, kq = l >> 4, u = (i >> 6) & 7;
+        const int p0 = 16 * (i >> 9);
+        const uint16_t *kr = (const uint16_t *)&ks[p0 + 4 * (m & 3) + (m >> 2)][0] + 16 * u + kq;
+        kt[i] = make_float4(h2f(kr[0]), h2f(kr[4]), h2f(kr[8]), h2f(kr[12]));
+        float v[4];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {   // vt[g][d]: dim d of positions 4g .. 4g+3
-        const int i = tid + 256 * k, g = i >> 7, d = i & (kHd - 1);
-        uint32_t v[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = ((const uint16_t *)&vs[4 * g + r][0])[d];
-        vt[i] = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
+        for (int e = 0; e < 4; ++e) v[e] = h2f(((const uint16_t *)&vs[p0 + 4 * e + kq][0])[16 * u + m]);
+        vt[i] = make_float4(v[0], v[1], v[2], v[3]);
     }
 }
 
-template <int G>
-__global__ __launch_bounds__(kPfmThreads) void attn_prefill_mfma_kernel(
-    const float *__restrict__ q, const float4 *__restrict__ Kt, const uint4 *__restrict__ Vt,
+// softmax_row_regs for a row in slot order (position 16J + 4j + k at slot
+// 16J + 4k + j): lane l's float4 of group jj holds positions 256jj + 16(l/4)
+// + 4i + l%4, i = 0..3, so thread t = 16(l/4) + 4i + l%4 of the 256-thread
+// workgroup sits in component i: its halving tree runs over lanes 32, 16, 8,
+// 4 apart (strides 128 .. 16), the components (8, 4), then lanes 2, 1 apart.
+// The row holds raw dots (scaled here, which makes them canonical, so the max
+// needs no extra instructions).  256 (NJ - 1) < S <= 256 NJ: only the last
+// group is masked.  In place; slots of positions >= S become zeros.
+template <int NJ>
+__device__ __forceinline__ void softmax_row_slots(float *row, float scale, int S, int Sw,
+                                                  int lane) {
+    float x[NJ][4];
+    const int t0 = 16 * (lane >> 2) + (lane & 3);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int at = 256 * j + 4 * lane;
+        const float4 v = *(const float4 *)(row + (j < NJ - 1 ? at : min(at, Sw - 4)));
+        x[j][0] = v.x * scale; x[j][1] = v.y * scale; x[j][2] = v.z * scale; x[j][3] = v.w * scale;
+    }
+    // past the row: no effect on the max, and exp(-inf - max) is exactly 0
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        x[NJ - 1][i] = 256 * (NJ - 1) + t0 + 4 * i < S ? x[NJ - 1][i] : -__builtin_inff();
+    float m = -3.402823e+38f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m = fmaxf(m, x[j][i]);
+    m = wave_max_dpp(m);
+    float c[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            x[j][i] = oxb_expf_nonpos(x[j][i] - m);
+            c[i] = c[i] + x[j][i];
+        }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float v = c[i];
+        v = v + __shfl_down(v, 32, 64);
+        v = v + __shfl_down(v, 16, 64);
+        v = v + __int_as_float(dpp0<0x108, 0xf>(__float_as_int(v)));
+        c[i] = v + __int_as_float(dpp0<0x104, 0xf>(__float_as_int(v)));
+    }
+    float sum = (c[0] + c[2]) + (c[1] + c[3]);
+    sum = sum + __int_as_float(dpp0<0x102, 0xf>(__float_as_int(sum)));
+    sum = sum + __int_as_float(dpp0<0x101, 0xf>(__float_as_int(sum)));
+    const float inv = 1.0f / __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sum), 0));
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int s0 = 256 * j + 4 * lane;
+        if (j < NJ - 1 || s0 < Sw)
+            *(float4 *)(row + s0) =
+                make_float4(x[j][0] * inv, x[j][1] * inv, x[j][2] * inv, x[j][3] * inv);
+    }
+}
+
+// softmax_row_slots for rows of up to 256 MAXJ positions
+template <int MAXJ, int NJ = 1>
+__device__ __forceinline__ void softmax_row_upto(float *row, float scale, int S, int Sw, int lane) {
+    if constexpr (NJ < MAXJ) {
+        if (S > 256 * NJ) return softmax_row_upto<MAXJ, NJ + 1>(row, scale, S, Sw, lane);
+    }
+    // opaque: nothing of one size is shared with another's or kept across rows
+    // (the registers would spill)
+    asm volatile("" : "+v"(lane));
+    softmax_row_slots<NJ>(row, scale, S, Sw, lane);
+}
+
+template <int G, int R>
+__global__ __launch_bounds__(kPfmThreads, R == 16 ? 4 : 2) void attn_prefill_mfma_kernel(
+    const float *__restrict__ q, const float4 *__restrict__ Kt, const float4 *__restrict__ Vt,
     int ntile_ws, int pos0, int n_q, int H, float scale, float *__restrict__ out) {
-    constexpr int QB = 16 / G;   // queries per workgroup
-    extern __shared__ __align__(16) float smem[];
-    float *qs = smem, *rows = smem + 16 * kPfmQs;
-    const int tid = threadIdx.x, lane = tid & 63;
+    constexpr int QB = R / G;   // queries per workgroup
+    constexpr int MAXS = R == 16 ? kPfmMaxS16 : kPfmMaxS8;
+    extern __shared__ __align__(16) float rows[];
+    const int tid = threadIdx.x, lane = tid & 63, kq = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform loop control
     const int nblk = (n_q + QB - 1) / QB, Hkv = H / G;
     // Block b runs on XCD b % 8.  A KV head's query blocks j (longest rows
@@ -1309,188 +1407,133 @@ __global__ __launch_bounds__(kPfmThreads) void attn_prefill_mfma_kernel(
     if (j >= nblk) return;   // the whole workgroup, before any barrier
     const int q0 = (nblk - 1 - j) * QB;
     const int Smax = pos0 + min(q0 + QB - 1, n_q - 1) + 1;
-    const int ntile = (Smax + 63) >> 6;
-    if (ntile > ntile_ws || Smax > kPfmMaxS) return;   // host checks too; never read out of range
+    if (((Smax + kKvTile - 1) / kKvTile) > ntile_ws || Smax > MAXS) return;   // host checks too
     const int Sw = pfm_row_stride(Smax);
     auto row_len = [&](int r) { return pos0 + min(q0 + r / G, n_q - 1) + 1; };
+    const int rl = lane & (R - 1);   // the score row of this lane's column
 
-    for (int i = tid; i < 16 * (kHd / 4); i += kPfmThreads) {
+    for (int i = tid; i < R * (kHd / 4); i += kPfmThreads) {
         const int r = i / (kHd / 4), c = i % (kHd / 4);
         const int qi = min(q0 + r / G, n_q - 1);
-        *(float4 *)(qs + r * kPfmQs + 4 * c) =
+        *(float4 *)(rows + r * kPfmQs + 4 * c) =
             *(const float4 *)(q + ((size_t)qi * H + hk * G + r % G) * kHd + 4 * c);
     }
+    const int nt = (Smax + 15) >> 4;   // 16-position tiles
+    const CopyRsrc kt = copy_rsrc(Kt, hk, ntile_ws);
+    // K steps (16 dims of a tile): the next tile's step takes the registers
+    // of a step once it is done, one load per step (four loads in one burst
+    // per 16 MFMAs hold the pipe to 2/3)
+    float4 kr[8];
+    auto loadk = [&](int u, int t) {
+        kr[u] = copy_load(kt, lane, min(t, nt - 1) * (kTileF4 * 16) + 1024 * u);
+    };
+    constexpr int NW = kPfmWaves;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) loadk(u, w);
     lds_barrier();
 
     // ---- scores (sh/attention.wgsl:48-58) ----------------------------------
     {
-        const float *qrow = qs + (lane & 15) * kPfmQs;
-        for (int t = w; t < ntile; t += kPfmWaves) {
-            const float4 *kt = Kt + ((size_t)hk * ntile_ws + t) * kTileF4 + lane;
-            v16f acc = {};
-            float4 kg[2][8];   // dims 32g .. 32g+31 of this lane's position, two groups
+        float4 qr[kHd / 16];   // component e of qr[u]: q[row][16u + 4e + kq]
 #pragma unroll
-            for (int j = 0; j < 8; ++j) kg[0][j] = kt[64 * j];
+        for (int u = 0; u < kHd / 16; ++u) {
+            const float *src = rows + rl * kPfmQs + 16 * u + kq;
+            qr[u] = make_float4(src[0], src[4], src[8], src[12]);
+        }
+        lds_barrier();       // every wave holds its q before the rows are written
+        for (int t = w; t < nt; t += NW) {
+            v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int g = 0; g < kHd / 32; ++g) {
-                if (g + 1 < kHd / 32) {
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) kg[(g + 1) & 1][j] = kt[64 * (8 * (g + 1) + j)];
-                }
-                __builtin_amdgcn_sched_barrier(0);   // next group's loads ahead of these MFMAs
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int c = 8 * g + j;   // dims 4c .. 4c+3
-                    const float4 qv = *(const float4 *)(qrow + 4 * c);
-                    const float4 kv = kg[g & 1][j];
-                    acc = mfma_f32_k1(qv.x, kv.x, acc);
-                    acc = mfma_f32_k1(qv.y, kv.y, acc);
-                    acc = mfma_f32_k1(qv.z, kv.z, acc);
-                    acc = mfma_f32_k1(qv.w, kv.w, acc);
-                }
+            for (int u = 0; u < 8; ++u) {
+                mfma_steps4(acc, kr[u], qr[u]);
+                __builtin_amdgcn_sched_barrier(0);
+                loadk(u, t + NW);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            const int r0 = 4 * (lane >> 4), p = 64 * t + (lane & 15);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int pos = p + 16 * (r >> 2);
-                if (pos < Smax) rows[(r0 + (r & 3)) * Sw + pos] = acc[r] * scale;
-            }
+            if (R == 16 || (lane & 15) < R)
+                *(float4 *)(rows + rl * Sw + 16 * t + 4 * kq) =
+                    make_float4(acc[0], acc[1], acc[2], acc[3]);
         }
     }
+    // V's first batches go out ahead of the softmax
+    const int len0 = row_len(0), s_end = Smax;   // lengths do not decrease in the row
+    const int nb = len0 >> 4, last = nt - 1;   // whole batches; the last one
+    const CopyRsrc vt = copy_rsrc(Vt, hk, ntile_ws);
+    constexpr int NV = kPvAhead + 1;
+    float4 vr[NV], vtail[2];
+    auto loadv = [&](float4 &v, int b) {
+        __builtin_amdgcn_sched_barrier(0);
+        v = copy_load(vt, lane, min(b, last) * (kTileF4 * 16) + 1024 * w);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int i = 0; i < NV - 1; ++i) loadv(vr[i], i);
+    loadv(vtail[0], nb);
+    loadv(vtail[1], nb + 1);
     lds_barrier();
 
     // ---- softmax (sh/softmax.wgsl:25-80) ------------------------------------
-    for (int r = w; r < 16; r += kPfmWaves) {
+    for (int r = w; r < R; r += kPfmWaves) {
         const int S = row_len(r);
-        // wave_softmax_row for rows of up to kPfmMaxS positions (register-held row)
         float *row = rows + r * Sw;
-        const int nj = (S + 255) >> 8;
-        if (nj <= 1) softmax_row_regs<1, true>(row, row, S, Sw, lane);
-        else if (nj <= 2) softmax_row_regs<2, true>(row, row, S, Sw, lane);
-        else if (nj <= 4) softmax_row_regs<4, true>(row, row, S, Sw, lane);
-        else if (nj <= 6) softmax_row_regs<6, true>(row, row, S, Sw, lane);
-        else if (nj <= 8) softmax_row_regs<8, true>(row, row, S, Sw, lane);
-        else softmax_row_regs<(kPfmMaxS + 255) / 256, true>(row, row, S, Sw, lane);
-        for (int s = S + lane; s < Sw; s += 64) row[s] = 0.0f;   // same wave: in order
+        softmax_row_upto<(MAXS + 255) / 256>(row, scale, S, Sw, lane);
     }
     lds_barrier();
 
     // ---- P.V (sh/attention.wgsl:96-104): one chain per output ---------------
-    if (w < 4) {
-        // wave w: rows 8(w&1) .. +7 as two groups of four (chains a and b,
-        // one V operand for both) x dims 64(w>>1) .. +63; lane l: dim d
-        const int r0 = 8 * (w & 1), d = 64 * (w >> 1) + lane;
-        int len[8];   // lengths non-decreasing in the row
-#pragma unroll
-        for (int i = 0; i < 8; ++i) len[i] = row_len(r0 + i);
-        const int e = len[0] & ~15;   // whole batches every row of the wave covers
-        const int s_end = len[7];
-        const int s_last = 64 * ntile - 16;   // last batch start inside Vt and the rows
-        const uint2 *vt = (const uint2 *)(Vt + (size_t)hk * ntile_ws * kVTileU4) + d;
-        const float *pa = rows + (r0 + (lane & 3)) * Sw, *pb = pa + 4 * Sw;
-        // 16 positions per batch: V (global) kPvAhead batches ahead in a ring
-        // of registers, p (LDS) at its batch (batch starts past the rows are
-        // clamped)
-        constexpr int NV = kPvAhead + 1;
-        uint2 vr[NV][4];
-        float4 qa[4], qb[4];
-        auto loadv = [&](uint2 (&vv)[4], int s) {
-            const int sb = min(s, s_last);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) vv[j] = vt[(size_t)(sb / 4 + j) * kHd];
-            __builtin_amdgcn_sched_barrier(0);
-        };
-        auto loadp = [&](int s) {
-            const int sb = min(s, s_last);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                qa[j] = *(const float4 *)(pa + sb + 4 * j);
-                qb[j] = *(const float4 *)(pb + sb + 4 * j);
-            }
-        };
-        auto vk = [](const uint2 &u, int k) {   // position k of the lane's quad
-            const uint32_t wd = k < 2 ? u.x : u.y;
-            return __half2float(__ushort_as_half((uint16_t)((k & 1) ? wd >> 16 : wd & 0xffffu)));
-        };
-        v4f a = {0.0f, 0.0f, 0.0f, 0.0f}, b = {0.0f, 0.0f, 0.0f, 0.0f};
-        // the batch's 16 V values converted first (while its p reads land),
-        // then its 32 steps back to back
-        auto run = [&](const uint2 (&vv)[4]) {
-            float vf[16];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) vf[i] = vk(vv[i >> 2], i & 3);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float pa4[4] = {qa[j].x, qa[j].y, qa[j].z, qa[j].w};
-                const float pb4[4] = {qb[j].x, qb[j].y, qb[j].z, qb[j].w};
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    a = __builtin_amdgcn_mfma_f32_4x4x1f32(pa4[k], vf[4 * j + k], a, 0, 0, 0);
-                    b = __builtin_amdgcn_mfma_f32_4x4x1f32(pb4[k], vf[4 * j + k], b, 0, 0, 0);
-                }
-            }
-        };
-        // the batch at st, each row's sum kept past its own length
-        auto tail = [&](const uint2 (&vv)[4], int st) {
-            if (st >= s_end) return;
-            loadp(st);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float pa4[4] = {qa[j].x, qa[j].y, qa[j].z, qa[j].w};
-                const float pb4[4] = {qb[j].x, qb[j].y, qb[j].z, qb[j].w};
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const int s = st + 4 * j + k;
-                    const float v = vk(vv[j], k);
-                    const v4f ra = __builtin_amdgcn_mfma_f32_4x4x1f32(pa4[k], v, a, 0, 0, 0);
-                    const v4f rb = __builtin_amdgcn_mfma_f32_4x4x1f32(pb4[k], v, b, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        a[i] = s < len[i] ? ra[i] : a[i];
-                        b[i] = s < len[4 + i] ? rb[i] : b[i];
-                    }
-                }
-            }
-        };
-        // batch n sits in vr[n % NV].  Passes of NV batches with no branch
-        // inside (ring indices are constants, and the loads stay in flight
-        // across batches), then the r < NV whole batches left, then the
-        // tails: batches r and r + 1 (the positions past e, fewer than 32)
-#pragma unroll
-        for (int i = 0; i < NV - 1; ++i) loadv(vr[i], 16 * i);
-        int s0 = 0;
-        for (; s0 + 16 * NV <= e; s0 += 16 * NV) {
-#pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                loadv(vr[(i + NV - 1) % NV], s0 + 16 * (i + NV - 1));
-                loadp(s0 + 16 * i);
-                run(vr[i]);
-            }
-        }
-        const int r = (e - s0) >> 4;
-#pragma unroll
-        for (int i = 0; i < NV - 1; ++i) {
-            if (i < r) {
-                loadv(vr[(i + NV - 1) % NV], s0 + 16 * (i + NV - 1));
-                loadp(s0 + 16 * i);
-                run(vr[i]);
-            }
-        }
+    const float *pr = rows + rl * Sw + 4 * kq;
+    v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    float4 p[2];   // read one batch ahead (the batch past the last one is never used)
+    p[0] = *(const float4 *)pr;
+    // batch b sits in vr[b % NV]: passes of NV batches with no branch inside
+    // (ring indices are constants and the loads stay in flight), then the
+    // whole batches left
+    int b0 = 0;
+    for (; b0 + NV <= nb; b0 += NV) {
+        const float *pb = pr + 16 * b0;
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            if (i == r) {
-                tail(vr[i], s0 + 16 * i);
-                tail(vr[(i + 1) % NV], s0 + 16 * (i + 1));
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int r = r0 + i, qi = q0 + r / G;
-            if (qi < n_q) out[((size_t)qi * H + hk * G + r % G) * kHd + d] = i < 4 ? a[i] : b[i - 4];
+            loadv(vr[(i + NV - 1) % NV], b0 + i + NV - 1);
+            p[(i + 1) & 1] = *(const float4 *)(pb + 16 * (i + 1));
+            mfma_steps4(acc, vr[i], p[i & 1]);
         }
     }
+    const float *pb = pr + 16 * b0;
+#pragma unroll
+    for (int i = 0; i < NV - 1; ++i)
+        if (b0 + i < nb) {
+            p[(i + 1) & 1] = *(const float4 *)(pb + 16 * (i + 1));
+            mfma_steps4(acc, vr[i], p[i & 1]);
+        }
+    // the last positions (fewer than 16 + QB), in groups of four
+    const int len = row_len(rl);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int s0 = 16 * (nb + h);
+        if (s0 >= s_end) break;
+        const float4 p4 = *(const float4 *)(pr + s0);
+        const float pt[4] = {p4.x, p4.y, p4.z, p4.w};
+        const float vv[4] = {vtail[h].x, vtail[h].y, vtail[h].z, vtail[h].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int s = s0 + 4 * e;
+            if (s + 4 <= len0) {
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[e], pt[e], acc, 0, 0, 0);
+            } else if (s < s_end) {
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) {
+                    const v4f r = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        kq == kk ? vv[e] : 0.0f, kq == kk ? pt[e] : -0.0f, acc, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[i] = s + kk < len ? r[i] : acc[i];
+                }
+            }
+        }
+    }
+    const int qi = q0 + rl / G;
+    if ((R == 16 || (lane & 15) < R) && qi < n_q)
+        *(float4 *)(out + ((size_t)qi * H + hk * G + rl % G) * kHd + 16 * w + 4 * kq) =
+            make_float4(acc[0], acc[1], acc[2], acc[3]);
 }
 
 // ---------------------------------------------------------------------------
@@ -2633,36 +2676,47 @@ static int launch_prefill_g(const float *q, const uint16_t *kc, const uint16_t *
     return launch_prefill<G, 1>(q, kc, vc, pos0, n_q, H, Hkv, max_seq, s_max, out, s);
 }
 
-template <int G>
-static int launch_prefill_mfma(const float *q, const uint16_t *kc, const uint16_t *vc, int pos0,
-                               int n_q, int H, int Hkv, int max_seq, int s_max, void *ws,
-                               float *out, hipStream_t s) {
-    constexpr int QB = 16 / G;
-    if (allow_dynamic_lds((const void *)attn_prefill_mfma_kernel<G>)) return -1;
-    const int ntile = (s_max + 63) / 64;
-    float4 *Kt = (float4 *)ws;
-    uint4 *Vt = (uint4 *)(Kt + (size_t)Hkv * ntile * kTileF4);
-    hipLaunchKernelGGL(attn_kv_tiles_kernel, dim3(ntile, Hkv), dim3(256), 0, s, kc, vc, max_seq,
-                       s_max, ntile, Kt, Vt);
-    OXB_CHECK_HIP(hipGetLastError());
+// 16-position tiles of the copies, rounded up to a whole pair
+static int kv_tiles(int s_max) { return 2 * ((s_max + 2 * kKvTile - 1) / (2 * kKvTile)); }
+
+template <int G, int R>
+static int launch_prefill_mfma_r(const float *q, const float4 *Kt, const float4 *Vt, int ntile,
+                                 int pos0, int n_q, int H, int Hkv, int s_max, float *out,
+                                 hipStream_t s) {
+    constexpr int QB = R / G;
+    if (allow_dynamic_lds((const void *)attn_prefill_mfma_kernel<G, R>)) return -1;
     const float scale = 1.0f / sqrtf((float)kHd);  // nn/attention.rs:206
-    hipLaunchKernelGGL((attn_prefill_mfma_kernel<G>), dim3(8 * Hkv * ((n_q + QB * 8 - 1) / (QB * 8))),
-                       dim3(kPfmThreads), pfm_smem(s_max), s, q, Kt, Vt, ntile, pos0, n_q, H,
-                       scale, out);
+    hipLaunchKernelGGL((attn_prefill_mfma_kernel<G, R>),
+                       dim3(8 * Hkv * ((n_q + QB * 8 - 1) / (QB * 8))), dim3(kPfmThreads),
+                       pfm_smem(R, s_max), s, q, Kt, Vt, ntile, pos0, n_q, H, scale, out);
     OXB_CHECK_HIP(hipGetLastError());
     return 0;
 }
 
-size_t attn_prefill_ws_bytes(int Hkv, int s_max) {
-    if (Hkv <= 0 || s_max <= 0 || s_max > kPfmMaxS) return 0;
-    return (size_t)Hkv * ((s_max + 63) / 64) * (kTileF4 * sizeof(float4) + kVTileU4 * sizeof(uint4));
+template <int G>
+static int launch_prefill_mfma(const float *q, const uint16_t *kc, const uint16_t *vc, int pos0,
+                               int n_q, int H, int Hkv, int max_seq, int s_max, void *ws,
+                               float *out, hipStream_t s) {
+    const int ntile = kv_tiles(s_max);
+    float4 *Kt = (float4 *)ws, *Vt = Kt + (size_t)Hkv * ntile * kTileF4;
+    hipLaunchKernelGGL(attn_kv_tiles_kernel, dim3(ntile / 2, Hkv), dim3(256), 0, s, kc, vc, max_seq,
+                       s_max, ntile, Kt, Vt);
+    OXB_CHECK_HIP(hipGetLastError());
+    if (s_max <= kPfmMaxS16)
+        return launch_prefill_mfma_r<G, 16>(q, Kt, Vt, ntile, pos0, n_q, H, Hkv, s_max, out, s);
+    return launch_prefill_mfma_r<G, 8>(q, Kt, Vt, ntile, pos0, n_q, H, Hkv, s_max, out, s);
 }
 
-size_t attn_prefill_ws_max_bytes(int Hkv) { return attn_prefill_ws_bytes(Hkv, kPfmMaxS); }
+size_t attn_prefill_ws_bytes(int Hkv, int s_max) {
+    if (Hkv <= 0 || s_max <= 0 || s_max > kPfmMaxS8) return 0;
+    return (size_t)Hkv * kv_tiles(s_max) * (2 * kTileF4 * sizeof(float4));
+}
 
-// f32 MFMA kernel (with its Kt / Vt workspace) while its 16 rows fit the LDS
-// (up to kPfmMaxS positions), else the VALU kernel: the same sums in the same
-// order either way
+size_t attn_prefill_ws_max_bytes(int Hkv) { return attn_prefill_ws_bytes(Hkv, kPfmMaxS8); }
+
+// f32 MFMA kernel (with its Kt / Vt workspace) while its 16 or 8 rows fit the
+// LDS (up to kPfmMaxS8 positions), else the VALU kernel: the same sums in the
+// same order either way
 int attn_prefill(const float *q, const uint16_t *kc, const uint16_t *vc, int n_q, int pos0, int H,
                  int Hkv, int hd, int max_seq, void *ws, size_t ws_bytes, float *out,
                  void *stream) {

@@ -596,6 +596,30 @@ def test_attn_prefill_causal_bitexact(H, Hkv, S, pos0, n):
     assert np.array_equal(out, ref)
 
 
+# Edges of the f32-MFMA prefill attention: its P.V runs 32 positions per batch,
+# then groups of four, then single steps where the rows' lengths differ, so
+# lengths sit on each side of 4, 16 and 32; rows past 2496 positions take 8
+# score rows per workgroup (up to 5056), longer ones the VALU kernel
+@pytest.mark.parametrize("H,Hkv,pos0,n", [(20, 5, 0, 2), (20, 5, 0, 33), (20, 5, 26, 7),
+                                          (20, 5, 31, 5), (8, 8, 15, 18), (16, 8, 60, 8),
+                                          (16, 2, 30, 3), (20, 5, 2490, 6), (20, 5, 2490, 7),
+                                          (8, 8, 2501, 10), (16, 2, 3070, 3), (4, 1, 5049, 7),
+                                          (4, 1, 5050, 7)])
+def test_attn_prefill_length_edges(H, Hkv, pos0, n):
+    rng = np.random.default_rng(77 + n + pos0)
+    hd, S = 128, pos0 + n
+    q = rng.standard_normal((n, H * hd)).astype(np.float32)
+    kc = (rng.standard_normal((Hkv, S, hd)) * 0.7).astype(np.float16)
+    vc = rng.standard_normal((Hkv, S, hd)).astype(np.float16)
+    # the last position holds values that would spoil any row it leaked into
+    vc[:, S - 1, 0::3] = np.inf
+    vc[:, S - 1, 1::3] = np.nan
+    out = ops.attn_prefill(q, kc, vc, n, pos0, H, Hkv, hd, S)
+    ref = _oracle_attn(q.reshape(-1), kc, vc, n, S, H, Hkv, hd).reshape(n, H * hd)
+    assert np.array_equal(out, ref, equal_nan=True)
+    assert np.isfinite(out[:-1]).all()
+
+
 # n > 64: the DMA-staged 256x128 kernel (8192 x 1024 with one K stage; 8192 x
 # 1000 and 8192 x 900 with 10 and 3 stages and a ragged last token tile), the
 # LDS-staged kernel at 128x128 (4224, 1024), 128x64 (6912, 512), 64x128 with a
