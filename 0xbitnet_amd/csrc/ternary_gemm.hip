@@ -324,12 +324,13 @@ __device__ __forceinline__ void gemm_stage_store(const u32x4_t (&rw)[WPT],
 }
 
 // One LDS stage of a wave's MF x MT tiles (wf, wt: its first row pair and
-// token pair in the workgroup; NF, NT: the workgroup's row and token pairs).
-template <int MF, int MT, int NF, int NT>
+// token pair in the workgroup; NF, NT: the workgroup's row and token pairs;
+// CP: chunk pairs of the stage, 2 for 256 k, 1 for 128).
+template <int MF, int MT, int NF, int NT, int CP = 2>
 __device__ __forceinline__ void gemm_mma_stage(v16i (&acc)[MF][MT], const uint4 *swb,
                                                const uint4 *sxb, int wf, int wt, int l) {
 #pragma unroll
-    for (int cp = 0; cp < 2; ++cp) {
+    for (int cp = 0; cp < CP; ++cp) {
         uint4 wu[MF];
 #pragma unroll
         for (int i = 0; i < MF; ++i) wu[i] = swb[(cp * NF + wf + i) * 64 + l];
@@ -340,7 +341,7 @@ __device__ __forceinline__ void gemm_mma_stage(v16i (&acc)[MF][MT], const uint4 
             for (int i = 0; i < MF; ++i) a[i] = plane(wu[i], g);
 #pragma unroll
             for (int j = 0; j < MT; ++j) {
-                const v4i bv = as_v4i(sxb[((g * 2 + cp) * NT + wt + j) * 64 + l]);
+                const v4i bv = as_v4i(sxb[((g * CP + cp) * NT + wt + j) * 64 + l]);
 #pragma unroll
                 for (int i = 0; i < MF; ++i)
                     acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[i], bv, acc[i][j], 0, 0, 0);
@@ -351,38 +352,45 @@ __device__ __forceinline__ void gemm_mma_stage(v16i (&acc)[MF][MT], const uint4 
 
 // Epilogue of the LDS-staged kernels: register v of tile (i, j) holds feature
 // 32(fp) + 8(v/4) + 4(l/32) + v%4 of token 32(tp) + l%32; stored as 4 groups
-// of 4 consecutive features, with every input loaded before the first store.
+// of 4 consecutive features, with the inputs of MG rows of tiles (all of
+// them, up to four tiles; a larger wave tile would not leave the registers)
+// loaded before their first store.
 template <int EPI, int MF, int MT>
 __device__ __forceinline__ void gemm_lds_epilogue(const GemmParams &p, const v16i (&acc)[MF][MT],
                                                   int ftile0, int ttile0, int wf, int wt, int l) {
+    constexpr int MG = MF * MT <= 4 ? MF : 1;
     EpiTok e[MT];
-    float4 ws[MF][4], old[MF][MT][4];
 #pragma unroll
     for (int j = 0; j < MT; ++j) e[j] = epi_tok<EPI>(p, (ttile0 + 2 * (wt + j)) * 16 + (l & 31));
 #pragma unroll
-    for (int i = 0; i < MF; ++i)
+    for (int i0 = 0; i0 < MF; i0 += MG) {
+        float4 ws[MG][4], old[MG][MT][4];
 #pragma unroll
-        for (int v4 = 0; v4 < 4; ++v4) {
-            const int n0 = (ftile0 + 2 * (wf + i)) * 16 + 8 * v4 + 4 * (l >> 5);
-            ws[i][v4] = *(const float4 *)(p.wscale + n0);
-#pragma unroll
-            for (int j = 0; j < MT; ++j)
-                old[i][j][v4] = epi_old<EPI>(p, (ttile0 + 2 * (wt + j)) * 16 + (l & 31), n0, e[j]);
-        }
-#pragma unroll
-    for (int i = 0; i < MF; ++i)
-#pragma unroll
-        for (int j = 0; j < MT; ++j) {
-            const int t = (ttile0 + 2 * (wt + j)) * 16 + (l & 31);
-            if (t >= p.n_tok) continue;
+        for (int i = 0; i < MG; ++i)
 #pragma unroll
             for (int v4 = 0; v4 < 4; ++v4) {
-                const v4i c = {acc[i][j][4 * v4], acc[i][j][4 * v4 + 1], acc[i][j][4 * v4 + 2],
-                               acc[i][j][4 * v4 + 3]};
-                gemm_store<EPI>(p, c, t, (ftile0 + 2 * (wf + i)) * 16 + 8 * v4 + 4 * (l >> 5), e[j],
-                                ws[i][v4], old[i][j][v4]);
+                const int n0 = (ftile0 + 2 * (wf + i0 + i)) * 16 + 8 * v4 + 4 * (l >> 5);
+                ws[i][v4] = *(const float4 *)(p.wscale + n0);
+#pragma unroll
+                for (int j = 0; j < MT; ++j)
+                    old[i][j][v4] = epi_old<EPI>(p, (ttile0 + 2 * (wt + j)) * 16 + (l & 31), n0, e[j]);
             }
-        }
+#pragma unroll
+        for (int i = 0; i < MG; ++i)
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                const int t = (ttile0 + 2 * (wt + j)) * 16 + (l & 31);
+                if (t >= p.n_tok) continue;
+#pragma unroll
+                for (int v4 = 0; v4 < 4; ++v4) {
+                    const v16i &r = acc[i0 + i][j];
+                    const v4i c = {r[4 * v4], r[4 * v4 + 1], r[4 * v4 + 2], r[4 * v4 + 3]};
+                    gemm_store<EPI>(p, c, t,
+                                    (ftile0 + 2 * (wf + i0 + i)) * 16 + 8 * v4 + 4 * (l >> 5), e[j],
+                                    ws[i][v4], old[i][j][v4]);
+                }
+            }
+    }
 }
 
 template <int EPI, int MF, int MT, int NWF>
@@ -467,25 +475,35 @@ __global__ __launch_bounds__(128 * NWF, 4 / NWF) void gemm_lds_kernel(GemmParams
 //   s+NBUF-1, multiply stage s.
 // (lds_dma16 and wait_vmcnt: oxb_common.h)
 
+// NWT: waves along the tokens.  CP = 1: stages of one chunk pair (128 k), half
+// the LDS per buffer, which is what lets
+// - 256 x 256 tiles (8 waves of 128 x 64, three 40 KB buffers) fit at all.
+//   A wave's LDS reads per MFMA fall from 0.63 to 0.38 KB and the workgroup
+//   stages a third less per output;
+// - 128 x 128 tiles (4 waves of 64 x 64, three 20 KB buffers) run two
+//   workgroups per CU, one's barriers and epilogue beside the other's MFMAs.
+// Both measured at gemm_launch.
+
 // workgroups per CU that the LDS of a DMA-staged tile allows (160 KB)
-__host__ __device__ constexpr int dma_occupancy(int MF, int MT, int NWF, int NBUF) {
-    return 160 * 1024 / (NBUF * (32 * NWF * MF * 4 + 64 * MT * 16) * 16) >= 2 ? 2 : 1;
+__host__ __device__ constexpr int dma_occupancy(int MF, int MT, int NWF, int NBUF, int NWT = 2,
+                                                int CP = 2) {
+    return 160 * 1024 / (NBUF * (32 * NWF * MF * 2 + 32 * NWT * MT * 8) * CP * 16) >= 2 ? 2 : 1;
 }
 
-template <int EPI, int MF, int MT, int NWF, int NBUF>
-__global__ __launch_bounds__(128 * NWF, dma_occupancy(MF, MT, NWF, NBUF)) void gemm_dma_kernel(
-    GemmParams p) {
-    constexpr int NTH = 128 * NWF;
-    constexpr int NF = NWF * MF, NT = 2 * MT;
+template <int EPI, int MF, int MT, int NWF, int NBUF, int NWT = 2, int CP = 2>
+__global__ __launch_bounds__(64 * NWF * NWT, dma_occupancy(MF, MT, NWF, NBUF, NWT, CP)) void
+gemm_dma_kernel(GemmParams p) {
+    constexpr int NTH = 64 * NWF * NWT;
+    constexpr int NF = NWF * MF, NT = NWT * MT;
     constexpr int FT = 32 * NF, TK = 32 * NT;
-    constexpr int WU = FT * 4, XU = TK * 16;
+    constexpr int WU = FT * 2 * CP, XU = TK * 8 * CP;
     constexpr int WPT = WU / NTH, XPT = XU / NTH, LPT = WPT + XPT;
     static_assert(WPT * NTH == WU && XPT * NTH == XU, "stage units must split evenly");
     static_assert(NBUF >= 3 && (NBUF - 2) * LPT < 64, "vmcnt holds the loads in flight");
     __shared__ uint4 sw[NBUF][WU];
     __shared__ uint4 sx[NBUF][XU];
     const int tid = threadIdx.x, l = tid & 63, w = tid >> 6;
-    const int KC = p.K >> 6, steps = KC >> 2;
+    const int KC = p.K >> 6, steps = KC / (2 * CP);
     const int ftile0 = blockIdx.x * (FT / 16), ttile0 = blockIdx.y * (TK / 16);
     const int ntt = (p.n_tok + 15) >> 4;
     const int wf = (w % NWF) * MF, wt = (w / NWF) * MT;
@@ -502,15 +520,16 @@ __global__ __launch_bounds__(128 * NWF, dma_occupancy(MF, MT, NWF, NBUF)) void g
 #pragma unroll
     for (int k = 0; k < XPT; ++k) {
         const int i = tid + NTH * k, u = i & 63, blk = i >> 6;
-        const int tp = blk % NT, gc = blk / NT, cp = gc & 1, g = gc >> 1, h = u >> 5;
+        const int tp = blk % NT, gc = blk / NT, cp = gc % CP, g = gc / CP, h = u >> 5;
         const int tt = min(ttile0 + 2 * tp + ((u >> 4) & 1), ntt - 1);
         xsrc[k] = p.X + (size_t)tt * KC * 64 + g * 64 + (2 * cp + h) * 16 + (u & 15);
     }
     auto issue = [&](int st, int b) {
+        const size_t xo = CP == 2 ? (size_t)st * 256 : (size_t)(st >> 1) * 256 + (st & 1) * 32;
 #pragma unroll
-        for (int k = 0; k < WPT; ++k) lds_dma16(wsrc[k] + (size_t)st * 64, sw[b] + NTH * k + 64 * w);
+        for (int k = 0; k < WPT; ++k) lds_dma16(wsrc[k] + (size_t)st * (32 * CP), sw[b] + NTH * k + 64 * w);
 #pragma unroll
-        for (int k = 0; k < XPT; ++k) lds_dma16(xsrc[k] + (size_t)st * 256, sx[b] + NTH * k + 64 * w);
+        for (int k = 0; k < XPT; ++k) lds_dma16(xsrc[k] + xo, sx[b] + NTH * k + 64 * w);
     };
     v16i acc[MF][MT];
 #pragma unroll
@@ -537,7 +556,7 @@ __global__ __launch_bounds__(128 * NWF, dma_occupancy(MF, MT, NWF, NBUF)) void g
         }
         lds_barrier();
         if (s + NBUF - 1 < steps) issue(s + NBUF - 1, b == 0 ? NBUF - 1 : b - 1);
-        gemm_mma_stage<MF, MT, NF, NT>(acc, sw[b], sx[b], wf, wt, l);
+        gemm_mma_stage<MF, MT, NF, NT, CP>(acc, sw[b], sx[b], wf, wt, l);
         b = b == NBUF - 1 ? 0 : b + 1;
     }
     gemm_lds_epilogue<EPI, MF, MT>(p, acc, ftile0, ttile0, wf, wt, l);
@@ -873,11 +892,12 @@ static int skinny_split_launch(const GemmParams &p, int pieces, void *ws, hipStr
     return 0;
 }
 
-template <int EPI, int MF, int MT, int NWF, int NBUF>
+template <int EPI, int MF, int MT, int NWF, int NBUF, int NWT = 2, int CP = 2>
 static int dma_launch(const GemmParams &p, hipStream_t s) {
-    constexpr int FT = 32 * MF * NWF, TK = 64 * MT;
+    constexpr int FT = 32 * MF * NWF, TK = 32 * MT * NWT;
     dim3 grid(p.N / FT, (p.n_tok + TK - 1) / TK);
-    hipLaunchKernelGGL((gemm_dma_kernel<EPI, MF, MT, NWF, NBUF>), grid, dim3(128 * NWF), 0, s, p);
+    hipLaunchKernelGGL((gemm_dma_kernel<EPI, MF, MT, NWF, NBUF, NWT, CP>), grid,
+                       dim3(64 * NWF * NWT), 0, s, p);
     OXB_CHECK_HIP(hipGetLastError());
     return 0;
 }
@@ -1003,8 +1023,28 @@ static int gemm_launch(const GemmParams &p, void *stream, void *ws = nullptr,
     // 64.4 / 33.6 us for 320 workgroups of 128x128).
     const int cus = device_cus();
     auto blocks = [&](int ft, int tk) { return (long)(p.N / ft) * ((p.n_tok + tk - 1) / tk); };
-    if (p.N % 256 == 0 && blocks(256, 128) >= cus * 5 / 8) return dma_launch<EPI, 2, 2, 4, 3>(p, s);
-    if (p.N % 128 == 0 && blocks(128, 128) >= cus) return lds_launch<EPI, 2, 2>(p, s);
+    // Once the 256x128 tiles (one per CU) need more than one round over the
+    // CUs, the last round is often nearly empty:
+    // - short rows (K < 4096, where a tile's pipeline fill and epilogue weigh
+    //   most): 128x128 tiles, two per CU.  K = 2560, us, 256x128 -> 128x128:
+    //   13824 rows at 600 / 1000 / 1500 / 2048 tokens 43.3 / 49.6 / 71.8 /
+    //   95.7 -> 39.2 / 47.2 / 67.6 / 83.5, 3840 at 2300 43.5 -> 37.3, 6912 at
+    //   2048 48.8 -> 47.3; one round is level (6912 at 1000 26.2 / 26.5);
+    // - long rows: 256x256 tiles, whose round costs 1.5-1.8 of a 256x128
+    //   round, where that saves time.  8192 x 28672 at 1500 / 2048 / 4001
+    //   tokens 361 / 401 / 1011 -> 331 / 381 / 757, 28672 x 8192 at 1500
+    //   340 -> 318, 5120 x 8192 at 2400 112 -> 102; where it does not:
+    //   8192 x 28672 at 2400 539 / 657, 28672 x 8192 at 2400 521 / 536.
+    // The 128x128 DMA-staged tile also replaced a register-staged one below 5/8
+    // of the CUs (2560 x 6912 at 1700 tokens 54.6 -> 48.7).
+    auto rounds = [&](long b) { return (b + cus - 1) / cus; };
+    if (p.N % 256 == 0 && blocks(256, 128) >= cus * 5 / 8) {
+        const long r = rounds(blocks(256, 128));
+        if (r > 1 && p.K < 4096) return dma_launch<EPI, 2, 2, 2, 3, 2, 1>(p, s);
+        if (9 * rounds(blocks(256, 256)) < 5 * r) return dma_launch<EPI, 4, 2, 2, 3, 4, 1>(p, s);
+        return dma_launch<EPI, 2, 2, 4, 3>(p, s);
+    }
+    if (p.N % 128 == 0 && blocks(128, 128) >= cus) return dma_launch<EPI, 2, 2, 2, 3, 2, 1>(p, s);
     if (p.N % 128 == 0 && blocks(128, 64) >= cus) return lds_launch<EPI, 2, 1>(p, s);
     if (p.N % 64 == 0 && blocks(64, 128) >= cus) return lds_launch<EPI, 1, 2>(p, s);
     if (p.N % 64 == 0) return dma_launch<EPI, 1, 1, 2, 4>(p, s);

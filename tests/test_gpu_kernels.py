@@ -660,6 +660,33 @@ def test_gemm_mfma_bitexact(N, K, n):
     assert np.array_equal(Y, Y_o)
 
 
+# Grids of more than one round over the CUs: 256x256 tiles for long rows (5 and
+# 6 token tiles, the last of 6 tokens or one; 14 of them over 10 feature
+# tiles), 128x128 tiles two per CU for short ones (one and ten K stages of 256,
+# ragged last tiles), and 128x128 where N is no multiple of 256.  Every epilogue,
+# on the rows at the tiles' edges and a few between
+@pytest.mark.parametrize("N,K,n", [(8192, 4096, 1030), (8192, 4096, 1281), (2560, 6912, 3330),
+                                   (13824, 256, 600), (3840, 2560, 2300), (4224, 512, 1030)])
+def test_gemm_large_grids_bitexact(N, K, n):
+    rng = np.random.default_rng(N + K + n)
+    Wn = synth.i2s_pack(ternary(rng, N, K))
+    x = rng.standard_normal((n, K)).astype(np.float32)
+    g = rng.uniform(0.5, 1.5, K).astype(np.float32)
+    ws = rng.uniform(0.01, 0.02, N).astype(np.float32)
+    r = rng.standard_normal((n, N)).astype(np.float32)
+    rows = sorted({t for b in range(0, n + 1, 128) for t in (b - 1, b) if 0 <= t < n} | {n - 1} |
+                  set(rng.integers(0, n, 8).tolist()))
+    q, s = O.quantize(O.rmsnorm(x[rows], g, 1e-5))
+    acc_o, Y_o = O.gemm(Wn, q, ws, s, K)
+    want = {0: Y_o, 1: O.add(r[rows], Y_o),
+            2: O.mul(O.relu2(Y_o[:, 0::2]), Y_o[:, 1::2])}
+    Wt = ops.upload_ternary(Wn, K)
+    for epi in (0, 1, 2):
+        acc, Y, _ = ops.gemm(Wt, x, g, 1e-5, ws, N, K, epilogue=epi, Y0=r if epi == 1 else None)
+        assert np.array_equal(acc[rows], acc_o), epi
+        assert np.array_equal(Y[rows], want[epi]), epi
+
+
 # the split GEMMs' arrival counters: a fixed area at the start of a workspace
 CNT_BYTES = 16384
 
