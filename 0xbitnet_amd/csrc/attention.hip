@@ -1259,8 +1259,15 @@ __host__ __device__ inline size_t pfm_smem(int R, int s_max) {
 // A KV head's copy as a buffer, read at a wave-uniform byte offset plus 16
 // bytes per lane: the address takes no VALU instruction, and nothing outside
 // the head's tiles can be read.
+// The descriptor has to be in scalar registers where a load is issued, or the
+// compiler wraps each load in a loop over the lanes' descriptors (eleven
+// instructions on the chains' path): readfirstlane keeps the head number
+// scalar.  Without it the form for one head per KV head (G = 1) shared the
+// number's widening with the divergent copy of the q rows (1 query of 2001
+// positions, 8 / 8 heads 59 us, with it 48).
 typedef __amdgpu_buffer_rsrc_t CopyRsrc;
 __device__ __forceinline__ CopyRsrc copy_rsrc(const float4 *copy, int hk, int ntile) {
+    hk = __builtin_amdgcn_readfirstlane(hk);
     return __builtin_amdgcn_make_buffer_rsrc(
         (void *)(copy + (size_t)hk * ntile * kTileF4), 0, ntile * kTileF4 * 16, 0x00027000);
 }

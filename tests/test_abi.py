@@ -5,7 +5,9 @@ No GPU compute is called here."""
 import ctypes as C
 import os
 import re
+import shutil
 import struct
+import subprocess
 
 import numpy as np
 import pytest
@@ -266,3 +268,30 @@ def test_gemm_workspace_sizes():
                   (8192, 28672, 4096), (2560, 2560, 8), (0, 256, 4), (100, 8192, 4),
                   (64, 8200, 4), (8192, 28672, 0)]:
         assert L.oxb_gemm_ws_bytes(*shape) == 0, shape
+
+
+def test_prefill_attention_reads_through_scalar_descriptors(tmp_path):
+    """Every form of the MFMA prefill attention holds its buffer descriptors in
+    scalar registers.  In vector registers each load becomes a loop with four
+    v_readfirstlane of its own, between the dependent MFMAs."""
+    objdump = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-objdump")
+    if not os.path.exists(objdump):
+        pytest.skip("no llvm-objdump")
+    lib = tmp_path / "liboxbitnet.so"
+    shutil.copy(os.path.join(ROOT, "0xbitnet_amd", "liboxbitnet.so"), lib)
+    run = lambda *a: subprocess.run([objdump, *a], check=True, capture_output=True, text=True,
+                                    cwd=tmp_path).stdout
+    run("--offloading", str(lib))   # the code objects, beside the copy
+    forms = {}
+    for obj in sorted(tmp_path.glob("*gfx950*")):
+        names = re.findall(r"\b(_ZN3oxb24attn_prefill_mfma_kernelILi\dELi\d+E\w+)$",
+                           run("-t", str(obj)), re.M)
+        if names:
+            asm = run("-d", "--disassemble-symbols=" + ",".join(names), str(obj))
+            for part in re.split(r"^[0-9a-f]+ <", asm, flags=re.M)[1:]:
+                forms[part.split(">")[0]] = part
+    assert len(forms) == 8   # 1, 2, 4, 8 heads per KV head x 16 and 8 rows
+    for name, asm in forms.items():
+        loads = len(re.findall(r"\bbuffer_load_dwordx4\b", asm))
+        assert loads >= 30, name
+        assert len(re.findall(r"\bv_readfirstlane_b32\b", asm)) < loads, name
