@@ -2721,9 +2721,32 @@ size_t attn_prefill_ws_bytes(int Hkv, int s_max) {
 
 size_t attn_prefill_ws_max_bytes(int Hkv) { return attn_prefill_ws_bytes(Hkv, kPfmMaxS8); }
 
+// Rows up to this long run on MFMA whatever the number of queries.
+constexpr int kPfmAlwaysS = 2368;
+
+// Past that, one or two heads per KV head and few queries: the VALU kernel,
+// which needs no copies, is the faster one while every workgroup has a CU of
+// its own and the K / V of the KV heads that one XCD's workgroups read (block b
+// runs on XCD b % 8) stay in its 4 MB L2; past that its K and V loads miss.
+// us, MFMA with its copies / VALU, G = 1, 8 KV heads: 1 query of 2420 positions
+// 54.7 / 45.6, 3 of 2420 54.9 / 47.0, 4 of 2420 (4.9 MB) 55.1 / 59.7, 3 of 2600
+// (4.0 MB) 54.9 / 54.0, 3 of 3000 61.4 / 84.4.  Past 2496 positions (8 rows per
+// workgroup) from four KV heads, whose copies weigh more (1 of 3000, G = 2: 8
+// KV heads 61.0 / 54.2, one 53.8 / 53.0), and up to 4096, past which the VALU
+// kernel's softmax leaves the registers (1 of 4600, G = 1, 8 KV heads 84.1 /
+// 95.6).  With more heads per KV head its chains run one after the other (1 of
+// 2401, G = 4, 8 KV heads 55.5 / 97.5).  Shorter rows would follow the same
+// line (1 of 1000, G = 1, 8 KV heads 26.1 / 20.7).
+static bool prefill_few_queries(int G, int Hkv, int n_q, int s_max) {
+    if (s_max <= kPfmAlwaysS || G > 2 || (long)n_q * Hkv > 256) return false;
+    const int heads = std::min(Hkv, (n_q * Hkv + 7) / 8);
+    return (size_t)heads * s_max * (2 * kHd * sizeof(uint16_t)) <= (4 << 20) &&
+           s_max <= (Hkv >= 4 ? 4096 : kPfmMaxS16);
+}
+
 // f32 MFMA kernel (with its Kt / Vt workspace) while its 16 or 8 rows fit the
-// LDS (up to kPfmMaxS8 positions), else the VALU kernel: the same sums in the
-// same order either way
+// LDS (up to kPfmMaxS8 positions) and there are more than a few queries, else
+// the VALU kernel: the same sums in the same order either way
 int attn_prefill(const float *q, const uint16_t *kc, const uint16_t *vc, int n_q, int pos0, int H,
                  int Hkv, int hd, int max_seq, void *ws, size_t ws_bytes, float *out,
                  void *stream) {
@@ -2733,7 +2756,7 @@ int attn_prefill(const float *q, const uint16_t *kc, const uint16_t *vc, int n_q
     const int G = H / Hkv, s_max = pos0 + n_q;
     hipStream_t s = (hipStream_t)stream;
     const size_t need = attn_prefill_ws_bytes(Hkv, s_max);
-    if (need && ws && ws_bytes >= need) {
+    if (need && ws && ws_bytes >= need && !prefill_few_queries(G, Hkv, n_q, s_max)) {
         switch (G) {
             case 1: return launch_prefill_mfma<1>(q, kc, vc, pos0, n_q, H, Hkv, max_seq, s_max, ws, out, s);
             case 2: return launch_prefill_mfma<2>(q, kc, vc, pos0, n_q, H, Hkv, max_seq, s_max, ws, out, s);
@@ -2958,7 +2981,10 @@ extern "C" int oxb_attn_prefill(const float *q, const uint16_t *kcache, const ui
     OXB_REQUIRE(H / Hkv == 1 || H / Hkv == 2 || H / Hkv == 4 || H / Hkv == 8,
                 "attention: GQA group %d unsupported (1, 2, 4, 8)", H / Hkv);
     hipStream_t s = (hipStream_t)stream;
-    const size_t need = attn_prefill_ws_bytes(Hkv, pos0 + n_tok);
+    const int s_max = pos0 + n_tok;
+    const size_t need = prefill_few_queries(H / Hkv, Hkv, n_tok, s_max)
+                            ? 0
+                            : attn_prefill_ws_bytes(Hkv, s_max);
     void *ws = nullptr;
     if (need) OXB_CHECK_HIP(hipMallocAsync(&ws, need, s));
     const int rc = attn_prefill(q, kcache, vcache, n_tok, pos0, H, Hkv, hd, max_seq, ws, need, out,

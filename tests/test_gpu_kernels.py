@@ -584,7 +584,15 @@ def test_attn_decode_fused_rejects_unsupported():
                                             (20, 5, 2368, 2300, 68),
                                             # VALU kernel: rows past 2368 positions
                                             (20, 5, 2600, 2369, 30), (16, 8, 3000, 2900, 17),
-                                            (8, 8, 2500, 2450, 11)])
+                                            (8, 8, 2500, 2450, 11),
+                                            # few queries of long rows with G = 1, 2: VALU at
+                                            # rows of 2369 or more, MFMA where the K / V of an
+                                            # XCD's workgroups pass 4 MB (4 of 2420, 5 of 3000)
+                                            (8, 8, 2368, 2366, 2), (8, 8, 2369, 2367, 2),
+                                            (8, 8, 2420, 2416, 4), (16, 8, 2604, 2601, 3),
+                                            (4, 4, 3000, 2995, 5), (32, 32, 2400, 2399, 1),
+                                            (16, 16, 4096, 4095, 1), (16, 16, 4097, 4096, 1),
+                                            (1, 1, 2500, 2490, 7), (2, 1, 2500, 2490, 6)])
 def test_attn_prefill_causal_bitexact(H, Hkv, S, pos0, n):
     rng = np.random.default_rng(21 + n)
     hd = 128
