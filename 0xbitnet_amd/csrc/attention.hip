@@ -2721,7 +2721,8 @@ size_t attn_prefill_ws_bytes(int Hkv, int s_max) {
 
 size_t attn_prefill_ws_max_bytes(int Hkv) { return attn_prefill_ws_bytes(Hkv, kPfmMaxS8); }
 
-// Rows up to this long run on MFMA whatever the number of queries.
+// Rows up to this long run on MFMA whatever the number of queries, and also
+// while a stream is captured.
 constexpr int kPfmAlwaysS = 2368;
 
 // Past that, one or two heads per KV head and few queries: the VALU kernel,
@@ -2969,8 +2970,16 @@ extern "C" int oxb_attn_decode_fused(const float *q, const uint16_t *kcache,
     }
 }
 
+static bool stream_captured(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) (void)hipGetLastError();
+    return st != hipStreamCaptureStatusNone;
+}
+
 // The Kt / Vt workspace is stream-ordered memory of this call (allocated and
-// released on the caller's stream).
+// released on the caller's stream).  A call that is being captured takes none
+// past kPfmAlwaysS positions: it runs on the VALU kernel, so that its graph
+// holds no allocation.
 extern "C" int oxb_attn_prefill(const float *q, const uint16_t *kcache, const uint16_t *vcache,
                                 int n_tok, int pos0, int H, int Hkv, int hd, int max_seq,
                                 float *out, void *stream) {
@@ -2982,9 +2991,10 @@ extern "C" int oxb_attn_prefill(const float *q, const uint16_t *kcache, const ui
                 "attention: GQA group %d unsupported (1, 2, 4, 8)", H / Hkv);
     hipStream_t s = (hipStream_t)stream;
     const int s_max = pos0 + n_tok;
-    const size_t need = prefill_few_queries(H / Hkv, Hkv, n_tok, s_max)
-                            ? 0
-                            : attn_prefill_ws_bytes(Hkv, s_max);
+    size_t need = prefill_few_queries(H / Hkv, Hkv, n_tok, s_max)
+                      ? 0
+                      : attn_prefill_ws_bytes(Hkv, s_max);
+    if (s_max > kPfmAlwaysS && need && stream_captured(s)) need = 0;
     void *ws = nullptr;
     if (need) OXB_CHECK_HIP(hipMallocAsync(&ws, need, s));
     const int rc = attn_prefill(q, kcache, vcache, n_tok, pos0, H, Hkv, hd, max_seq, ws, need, out,

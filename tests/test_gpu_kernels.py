@@ -6,6 +6,8 @@ attention and LM-head sums (different reduction order by design, f16 KV) are
 compared with an explicit tolerance, tighter than the 1e-3 relative bound
 the path is held to.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -626,6 +628,45 @@ def test_attn_prefill_length_edges(H, Hkv, pos0, n):
     ref = _oracle_attn(q.reshape(-1), kc, vc, n, S, H, Hkv, hd).reshape(n, H * hd)
     assert np.array_equal(out, ref, equal_nan=True)
     assert np.isfinite(out[:-1]).all()
+
+
+# A captured call past 2368 positions allocates nothing (VALU kernel: query
+# pairs, one query of 8 heads, one of one head): replayed with other q, eager
+# calls between the replays
+@pytest.mark.parametrize("H,Hkv,pos0,n", [(20, 5, 2600, 9), (16, 2, 4600, 3), (8, 8, 2500, 20)])
+def test_attn_prefill_captured(H, Hkv, pos0, n):
+    rng = np.random.default_rng([pos0, n])
+    hd, S = 128, pos0 + n
+    kc = (rng.standard_normal((Hkv, S, hd)) * 0.7).astype(np.float16)
+    vc = rng.standard_normal((Hkv, S, hd)).astype(np.float16)
+    L = ops.lib()
+    dq = ops.DeviceArray((n, H * hd), np.float32, zero=True)
+    dk, dv = (ops.DeviceArray.from_host(c.view(np.uint16)) for c in (kc, vc))
+    out = ops.DeviceArray((n, H * hd), np.float32, zero=True)
+    stream = L.oxb_stream_create()
+
+    def capture():
+        ops.check(L.oxb_stream_begin_capture(stream), "capture")
+        ops.check(L.oxb_attn_prefill(dq.ptr, dk.ptr, dv.ptr, n, pos0, H, Hkv, hd, S, out.ptr,
+                                     stream), "attn_prefill")
+
+    capture()   # one node, the kernel (dlsym also searches the linked HIP runtime)
+    g, nodes = C.c_void_p(), C.c_size_t()
+    assert L.hipStreamEndCapture(C.c_void_p(stream), C.byref(g)) == 0
+    assert L.hipGraphGetNodes(g, None, C.byref(nodes)) == 0 and nodes.value == 1
+    assert L.hipGraphDestroy(g) == 0
+    capture()
+    graph = L.oxb_stream_end_capture(stream)
+    assert graph
+    for _ in range(3):
+        q = rng.standard_normal((n, H * hd)).astype(np.float32)
+        dq.upload(q)
+        ops.sync()
+        ops.check(L.oxb_graph_launch(graph, stream), "replay")
+        ops.check(L.oxb_stream_sync(stream), "sync")
+        assert np.array_equal(out.download(), ops.attn_prefill(q, kc, vc, n, pos0, H, Hkv, hd, S))
+    L.oxb_graph_destroy(graph)
+    L.oxb_stream_destroy(stream)
 
 
 # n > 64: the DMA-staged 256x128 kernel (8192 x 1024 with one K stage; 8192 x
