@@ -261,8 +261,9 @@ int oxb_attn_decode_noalloc(const float *q, const uint16_t *kcache, const uint16
 
 /* Causal prefill attention for n_tok queries at positions pos0.., same order.
  * q, out: [n_tok][H*128] f32.  Replaces the same three dispatches for n > 1.
- * Up to 5056 positions the call takes a stream-ordered workspace of 1 KB per
- * position and KV head; under stream capture only up to 2368 positions. */
+ * Up to 5056 positions the call takes a workspace of 1 KB per position and KV
+ * head from a stream-ordered pool (up to 192 MB of which stay with the library
+ * per device); under stream capture only up to 2368 positions. */
 int oxb_attn_prefill(const float *q, const uint16_t *kcache, const uint16_t *vcache, int n_tok,
                      int pos0, int H, int Hkv, int hd, int max_seq, float *out, void *stream);
 

@@ -7,6 +7,7 @@ compared with an explicit tolerance, tighter than the 1e-3 relative bound
 the path is held to.
 """
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -667,6 +668,73 @@ def test_attn_prefill_captured(H, Hkv, pos0, n):
         assert np.array_equal(out.download(), ops.attn_prefill(q, kc, vc, n, pos0, H, Hkv, hd, S))
     L.oxb_graph_destroy(graph)
     L.oxb_stream_destroy(stream)
+
+
+def _free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()   # dlsym also searches the linked HIP runtime
+    assert ops.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_attn_prefill_workspace_is_kept_and_bounded():
+    """The workspace of a synchronized call stays for the next one (taking it
+    again costs more than a short call), 192 MB at the most once a call after a
+    larger one has ended."""
+    L, hd, H, S_max, n = ops.lib(), 128, 64, 5056, 5
+    arrs = [ops.DeviceArray((m,), np.float32, zero=True)
+            for m in (n * H * hd, H * S_max * hd // 2, H * S_max * hd // 2, n * H * hd)]
+    q, kc, vc, out = (a.ptr for a in arrs)
+    start = _free_bytes()
+
+    def taken(heads, S):
+        ops.check(L.oxb_attn_prefill(q, kc, vc, n, S - n, heads, heads, hd, S, out, None),
+                  "attn_prefill")
+        ops.sync()
+        return (start - _free_bytes()) / (1 << 20)
+
+    kept = taken(64, 3005)   # 188 MB of copies
+    assert 188 <= kept < 208
+    assert abs(taken(64, 3005) - kept) < 1
+    for S in (300, 5005, 2000, 5005, 100):   # 5005: 312 MB
+        kept = taken(64, S)
+        assert kept < 208 or S == 5005, S
+
+
+def test_attn_prefill_streams_and_threads():
+    """Calls of different lengths on four threads' streams at once."""
+    rng = np.random.default_rng(6)
+    L, H, Hkv, hd = ops.lib(), 20, 5, 128
+    jobs = []
+    for pos0, n in ((300, 40), (900, 70), (1700, 33), (2600, 12)):
+        S = pos0 + n
+        q = rng.standard_normal((n, H * hd)).astype(np.float32)
+        kc = (rng.standard_normal((Hkv, S, hd)) * 0.7).astype(np.float16)
+        vc = rng.standard_normal((Hkv, S, hd)).astype(np.float16)
+        jobs.append((pos0, n, S, ops.attn_prefill(q, kc, vc, n, pos0, H, Hkv, hd, S),
+                     [ops.DeviceArray.from_host(a) for a in (q, kc.view(np.uint16),
+                                                             vc.view(np.uint16))]))
+    errors = []
+
+    def work(job):
+        pos0, n, S, want, (q, kc, vc) = job
+        try:
+            stream = L.oxb_stream_create()
+            for rep in range(20):
+                out = ops.DeviceArray((n, H * hd), np.float32, zero=True)
+                ops.check(L.oxb_attn_prefill(q.ptr, kc.ptr, vc.ptr, n, pos0, H, Hkv, hd, S, out.ptr,
+                                             stream), "attn_prefill")
+                ops.check(L.oxb_stream_sync(stream), "sync")
+                assert np.array_equal(out.download(), want), (pos0, rep)
+            L.oxb_stream_destroy(stream)
+        except Exception as e:   # noqa: BLE001 - reported by the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(j,)) for j in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
 
 
 # n > 64: the DMA-staged 256x128 kernel (8192 x 1024 with one K stage; 8192 x
