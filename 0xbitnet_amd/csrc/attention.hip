@@ -2719,7 +2719,9 @@ size_t attn_prefill_ws_bytes(int Hkv, int s_max) {
     return (size_t)Hkv * kv_tiles(s_max) * (2 * kTileF4 * sizeof(float4));
 }
 
-size_t attn_prefill_ws_max_bytes(int Hkv) { return attn_prefill_ws_bytes(Hkv, kPfmMaxS8); }
+size_t attn_prefill_ws_max_bytes(int Hkv, int max_seq) {
+    return attn_prefill_ws_bytes(Hkv, max_seq < kPfmMaxS8 ? max_seq : kPfmMaxS8);
+}
 
 // Rows up to this long run on MFMA whatever the number of queries, and also
 // while a stream is captured.

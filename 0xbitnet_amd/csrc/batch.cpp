@@ -149,6 +149,7 @@ extern "C" oxb_batch *oxb_batch_create(oxb_model *m, int batch, int max_seq) {
         set_error("batch: %d positions exceed the attention LDS budget", max_seq);
         return nullptr;
     }
+    if (m->reserve_prefill_ws(max_seq)) return nullptr;
     oxb_batch *b = new oxb_batch;
     b->m = m;
     b->B = batch;

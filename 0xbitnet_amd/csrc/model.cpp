@@ -517,17 +517,14 @@ oxb_model *model_load(const char *path, int max_seq, LoadHook hook, void *ud, in
         }
     }
     m->tok_hist = (int *)m->dalloc((size_t)m->hist_cap * 4);
-    // the prefill attention's K / V copies, once, for the longest rows any
-    // prefill of this model or a batch slot can hand the MFMA kernel
-    m->pf_ws_bytes = oxb::attn_prefill_ws_max_bytes(Hkv);
-    m->pf_ws = m->dalloc(m->pf_ws_bytes);
+    if (m->reserve_prefill_ws(m->max_seq)) return nullptr;
     m->samp_ctl = (oxb::SampleCtl *)m->dalloc(sizeof(oxb::SampleCtl));
     m->samp_u = (float *)m->dalloc((size_t)m->hist_cap * 4);
     m->samp_ws_bytes = oxb::sample_ws_bytes(m->V);
     m->samp_ws = m->dalloc(m->samp_ws_bytes);
     if (!m->kcache || !m->vcache || (kv8_bytes && !m->vcache8) || !m->x || !m->q || !m->attn ||
         !m->h || !m->scores ||
-        !m->logits || !m->state || !m->tok_hist || !m->pf_ws || !m->samp_ctl || !m->samp_u ||
+        !m->logits || !m->state || !m->tok_hist || !m->samp_ctl || !m->samp_u ||
         !m->samp_ws || (m->qkv_attn && !m->qa_cnt))
         return nullptr;
     if ((m->qa_cnt && hipMemset(m->qa_cnt, 0, (size_t)H * 4) != hipSuccess) ||
@@ -694,6 +691,24 @@ int oxb_model::ensure_prefill(int n) {
     if (!nx || !nq || !na || !nh || !ns || !nX || !nsum || !nids) return -1;
     px = nx; pq = nq; pattn = na; ph = nh; pscale = ns; pX = nX; psum = nsum; pids = nids;
     pf_cap = cap;
+    return 0;
+}
+
+// The prefill attention's K / V copies for the longest rows that a cache of
+// max_seq positions can hand the MFMA kernel: taken when the model is loaded
+// and when a batch is created (whose slots may be longer than the model's own
+// cache), so that no prefill allocates.  The f32 cache's attention has none.
+int oxb_model::reserve_prefill_ws(int max_seq) {
+    const size_t need = kv_f32 ? 0 : oxb::attn_prefill_ws_max_bytes(Hkv, max_seq);
+    if (need <= pf_ws_bytes) return 0;
+    void *w = dalloc(need);
+    if (!w) return -1;
+    if (pf_ws) {   // released once the work queued on it is done
+        M_CHECK(hipStreamSynchronize(stream));
+        dfree(pf_ws);
+    }
+    pf_ws = w;
+    pf_ws_bytes = need;
     return 0;
 }
 

@@ -46,7 +46,7 @@ struct oxb_model {
 
     // prefill buffers (grown on demand)
     int pf_cap = 0;
-    void *pf_ws = nullptr;   // prefill attention's K / V copies (sized at load)
+    void *pf_ws = nullptr;   // prefill attention's K / V copies (reserve_prefill_ws)
     size_t pf_ws_bytes = 0;
     // the prefill GEMMs' split-K workspace (grown to the largest need met so
     // far; its arrival counters are zero between calls)
@@ -105,6 +105,7 @@ struct oxb_model {
     int enqueue_sample();   // the sampler over logits (state, history, draws)
     int ensure_prefill(int n);
     int ensure_gemm_ws(int n);
+    int reserve_prefill_ws(int max_seq);
     // one sequence's caches ([L][Hkv][max_seq][hd] each), RoPE table, state
     // block, token history and position
     struct SeqTarget {

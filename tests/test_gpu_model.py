@@ -625,3 +625,35 @@ def test_batch_rejects_unprefilled_slot():
         b.prefill(1, np.array([5], np.int32))
     b.close()
     m.close()
+
+
+def test_prefill_workspace_follows_the_context():
+    """The prefill attention's workspace is sized by the model's context (4 KV
+    heads: 20 MB for the longest rows the kernel takes, 256 KB for 64), and a
+    batch whose slots are longer than the model's cache gets what its own rows
+    need."""
+    cfg = synth.small_config(n_layers=1, kv_heads=4, context=4096)
+    path = synth.cached_gguf(cfg, seed=31)
+    L = pkg.lib()   # dlsym also searches the HIP runtime it is linked to
+
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert L.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    pkg.Model(path, max_seq=64).close()   # the runtime's own first allocations
+    before = free_bytes()
+    m = pkg.Model(path, max_seq=64)
+    assert before - free_bytes() < 14 << 20
+    ids = np.random.default_rng(31).integers(0, cfg.vocab, 2600).astype(np.int32)
+    m.forward(ids[:40])
+    b = pkg.Batch(m, 1, 2700)
+    ref = pkg.Model(path, max_seq=2700)
+    tok, _ = ref.forward(ids)
+    assert b.prefill(0, ids) == tok
+    steps = [ref.step() for _ in range(3)]
+    assert b.decode_greedy(3)[0].tolist() == [t for t, _ in steps]
+    _same(b.logits()[0], steps[-1][1], "slot")
+    b.close()
+    m.close()
+    ref.close()
