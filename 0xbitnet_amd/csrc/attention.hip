@@ -1241,6 +1241,9 @@ __global__ __launch_bounds__(kPrefillThreads) void attn_prefill_kernel(
 // SIMD the softmax's VALU time adds to the MFMA time whatever overlaps.
 // ---------------------------------------------------------------------------
 typedef float v4f __attribute__((ext_vector_type(4)));
+// Four floats of q or out, which callers need only align as floats (one
+// dwordx4 access either way).
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int kPfmWaves = 8;
 constexpr int kPfmThreads = 64 * kPfmWaves;
 constexpr int kPfmQs = kHd + 4;          // q row stride (floats)
@@ -1422,8 +1425,8 @@ __global__ __launch_bounds__(kPfmThreads, R == 16 ? 4 : 2) void attn_prefill_mfm
     for (int i = tid; i < R * (kHd / 4); i += kPfmThreads) {
         const int r = i / (kHd / 4), c = i % (kHd / 4);
         const int qi = min(q0 + r / G, n_q - 1);
-        *(float4 *)(rows + r * kPfmQs + 4 * c) =
-            *(const float4 *)(q + ((size_t)qi * H + hk * G + r % G) * kHd + 4 * c);
+        *(v4f *)(rows + r * kPfmQs + 4 * c) =
+            *(const v4f_any *)(q + ((size_t)qi * H + hk * G + r % G) * kHd + 4 * c);
     }
     const int nt = (Smax + 15) >> 4;   // 16-position tiles
     const CopyRsrc kt = copy_rsrc(Kt, hk, ntile_ws);
@@ -1539,8 +1542,7 @@ __global__ __launch_bounds__(kPfmThreads, R == 16 ? 4 : 2) void attn_prefill_mfm
     }
     const int qi = q0 + rl / G;
     if ((R == 16 || (lane & 15) < R) && qi < n_q)
-        *(float4 *)(out + ((size_t)qi * H + hk * G + rl % G) * kHd + 16 * w + 4 * kq) =
-            make_float4(acc[0], acc[1], acc[2], acc[3]);
+        *(v4f_any *)(out + ((size_t)qi * H + hk * G + rl % G) * kHd + 16 * w + 4 * kq) = acc;
 }
 
 // ---------------------------------------------------------------------------

@@ -737,6 +737,28 @@ def test_attn_prefill_streams_and_threads():
     assert not errors, errors
 
 
+# q and out need no more than a float's alignment, for 16 and for 8 score rows
+# per workgroup, and nothing is written past out
+@pytest.mark.parametrize("pos0", [30, 2500])
+def test_attn_prefill_float_aligned(pos0):
+    H, Hkv, hd, n = 20, 5, 128, 9
+    S = pos0 + n
+    rng = np.random.default_rng(pos0)
+    q = rng.standard_normal((n, H * hd)).astype(np.float32)
+    kc = (rng.standard_normal((Hkv, S, hd)) * 0.7).astype(np.float16)
+    vc = rng.standard_normal((Hkv, S, hd)).astype(np.float16)
+    dq = ops.DeviceArray.from_host(np.concatenate([np.zeros(1, np.float32), q.reshape(-1)]))
+    dk, dv = (ops.DeviceArray.from_host(c.view(np.uint16)) for c in (kc, vc))
+    out = ops.DeviceArray.from_host(np.full(n * H * hd + 2, 7.5, np.float32))
+    ops.check(ops.lib().oxb_attn_prefill(dq.offset(4), dk.ptr, dv.ptr, n, pos0, H, Hkv, hd, S,
+                                         out.offset(4), None), "attn_prefill")
+    ops.sync()
+    got = out.download()
+    ref = _oracle_attn(q.reshape(-1), kc, vc, n, S, H, Hkv, hd)
+    assert np.array_equal(got[1:-1], ref.reshape(-1))
+    assert got[0] == 7.5 and got[-1] == 7.5
+
+
 # n > 64: the DMA-staged 256x128 kernel (8192 x 1024 with one K stage; 8192 x
 # 1000 and 8192 x 900 with 10 and 3 stages and a ragged last token tile), the
 # LDS-staged kernel at 128x128 (4224, 1024), 128x64 (6912, 512), 64x128 with a
