@@ -493,6 +493,7 @@ __host__ __device__ constexpr int dma_occupancy(int MF, int MT, int NWF, int NBU
 template <int EPI, int MF, int MT, int NWF, int NBUF, int NWT = 2, int CP = 2>
 __global__ __launch_bounds__(64 * NWF * NWT, dma_occupancy(MF, MT, NWF, NBUF, NWT, CP)) void
 gemm_dma_kernel(GemmParams p) {
+    static_assert(CP == 1 || CP == 2, "stages of 128 or 256 k");
     constexpr int NTH = 64 * NWF * NWT;
     constexpr int NF = NWF * MF, NT = NWT * MT;
     constexpr int FT = 32 * NF, TK = 32 * NT;
@@ -503,7 +504,10 @@ gemm_dma_kernel(GemmParams p) {
     __shared__ uint4 sw[NBUF][WU];
     __shared__ uint4 sx[NBUF][XU];
     const int tid = threadIdx.x, l = tid & 63, w = tid >> 6;
-    const int KC = p.K >> 6, steps = KC / (2 * CP);
+    // K / (128 CP).  Each form as the compiler schedules the stages best, us: the
+    // shift for 256 k (4096 x 4096 at 1700 tokens 33.7, divided 34.5), the
+    // division for 128 (8192 x 28672 at 1500 tokens 311, shifted 317).
+    const int KC = p.K >> 6, steps = CP == 2 ? KC >> 2 : KC / 2;
     const int ftile0 = blockIdx.x * (FT / 16), ttile0 = blockIdx.y * (TK / 16);
     const int ntt = (p.n_tok + 15) >> 4;
     const int wf = (w % NWF) * MF, wt = (w / NWF) * MT;
