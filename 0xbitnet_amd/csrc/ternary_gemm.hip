@@ -1020,31 +1020,41 @@ static int gemm_launch(const GemmParams &p, void *stream, void *ws = nullptr,
                                  : two ? skinny_launch<EPI, 4, 2>(p, s) : skinny_launch<EPI, 4, 1>(p, s);
         }
     }
-    // LDS-staged tiles: the largest of 128x128, 128x64, 64x128, 64x64 whose
-    // grid still gives every CU a workgroup (N a multiple of the tile); the
-    // 256x128 DMA-staged tile already from 5/8 of the CUs (N = 2560 at 2048
-    // tokens, 160 workgroups: K = 6912 / 2560 take 56.3 / 29.2 us against
-    // 64.4 / 33.6 us for 320 workgroups of 128x128).
+    // Tiles staged through LDS: the largest of 128x128, 128x64, 64x128, 64x64
+    // whose grid still gives every CU a workgroup (N a multiple of the tile);
+    // 256x128 already from 5/8 of the CUs.  us, 256x128 / 128x128: 160
+    // workgroups of 256x128 (2560 rows at 2048 tokens) K = 6912 45.1 / 48.2, K =
+    // 2560 22.2 / 22.7; 140 (1700 tokens) 43.8 / 46.9, with the residual at K =
+    // 2560 26.8 / 26.2; 128, which leave each CU one 128x128 tile (4096 x 4096 at
+    // 1000 tokens) 29.7 / 24.5.
     const int cus = device_cus();
     auto blocks = [&](int ft, int tk) { return (long)(p.N / ft) * ((p.n_tok + tk - 1) / tk); };
     // Once the 256x128 tiles (one per CU) need more than one round over the
     // CUs, the last round is often nearly empty:
     // - short rows (K < 4096, where a tile's pipeline fill and epilogue weigh
-    //   most): 128x128 tiles, two per CU.  K = 2560, us, 256x128 -> 128x128:
-    //   13824 rows at 600 / 1000 / 1500 / 2048 tokens 43.3 / 49.6 / 71.8 /
-    //   95.7 -> 39.2 / 47.2 / 67.6 / 83.5, 3840 at 2300 43.5 -> 37.3, 6912 at
-    //   2048 48.8 -> 47.3; one round is level (6912 at 1000 26.2 / 26.5);
-    // - long rows: 256x256 tiles, whose round costs 1.5-1.8 of a 256x128
-    //   round, where that saves time.  8192 x 28672 at 1500 / 2048 / 4001
-    //   tokens 361 / 401 / 1011 -> 331 / 381 / 757, 28672 x 8192 at 1500
-    //   340 -> 318, 5120 x 8192 at 2400 112 -> 102; where it does not:
-    //   8192 x 28672 at 2400 539 / 657, 28672 x 8192 at 2400 521 / 536.
-    // The 128x128 DMA-staged tile also replaced a register-staged one below 5/8
-    // of the CUs (2560 x 6912 at 1700 tokens 54.6 -> 48.7).
+    //   most): 128x128 tiles, two per CU, whose rounds also end in halves.
+    //   us, 256x128 / 128x128, K = 2560: 13824 rows at 600 / 1500 / 2048 tokens
+    //   39.4 / 35.2, 64.6 / 62.2, 88.6 / 76.3, 3840 at 2400 41.1 / 35.4; K =
+    //   3584, 8192 rows at 1500 / 3000 53.8 / 46.7, 90.8 / 87.6.  Where a second
+    //   round has no half to save, 256x256 (next) is ahead of both: K = 2560,
+    //   13824 rows at 1000 45.2 / 44.3 / 42.0, K = 3584, 8192 at 1700 55.4 /
+    //   57.0 / 52.7;
+    // - 256x256 tiles, whose round costs 1.8 to 2 of a 256x128 round, where they
+    //   need about half the rounds.  us, 256x128 / 256x256: 8192 x 28672 at 1500
+    //   / 2048 / 4001 tokens 342 / 325, 377 / 361, 755 / 719, 28672 x 8192 at
+    //   1500 327 / 315, 5120 x 8192 at 2400 106 / 102.  6 rounds of 11 are in
+    //   between (22016 x 4096 at 4001 391 / 375, 28672 x 8192 at 3000 661 / 672),
+    //   3 of 5 and 5 of 9 no longer pay (13824 x 5120 at 2400 180 / 201, 28672 x
+    //   8192 at 2400 514 / 559).
+    // Longer rows leave the first rule out: 128x128 gains there too where a half
+    // is saved early (12288 x 4096 at 1000 59.4 / 52.0, 256x256 56.1), but loses
+    // late (28672 x 8192 at 3000 652 / 669).
     auto rounds = [&](long b) { return (b + cus - 1) / cus; };
     if (p.N % 256 == 0 && blocks(256, 128) >= cus * 5 / 8) {
         const long r = rounds(blocks(256, 128));
-        if (r > 1 && p.K < 4096) return dma_launch<EPI, 2, 2, 2, 3, 2, 1>(p, s);
+        // (two rounds of 256x128: three or four halves of 128x128)
+        if (p.K < 4096 && (r > 2 || (r == 2 && rounds(blocks(128, 128)) == 3)))
+            return dma_launch<EPI, 2, 2, 2, 3, 2, 1>(p, s);
         if (9 * rounds(blocks(256, 256)) < 5 * r) return dma_launch<EPI, 4, 2, 2, 3, 4, 1>(p, s);
         return dma_launch<EPI, 2, 2, 4, 3>(p, s);
     }

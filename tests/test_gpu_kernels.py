@@ -760,8 +760,8 @@ def test_attn_prefill_float_aligned(pos0):
 
 
 # n > 64: the DMA-staged 256x128 kernel (8192 x 1024 with one K stage; 8192 x
-# 1000 and 8192 x 900 with 10 and 3 stages and a ragged last token tile), the
-# LDS-staged kernel at 128x128 (4224, 1024), 128x64 (6912, 512), 64x128 with a
+# 1000 and 8192 x 900 with 10 and 3 stages and a ragged last token tile) and
+# 128x128 kernel (4224, 1024), the register-staged kernel at 128x64 (6912, 512), 64x128 with a
 # ragged last token tile (4032, 650), the DMA-staged 64x64 kernel with 4
 # buffers (2560 x 512 with 27 stages; 2 and 3 stages, fewer than it prefetches,
 # with ragged token tiles) -- and the register-tiled kernel for N % 64 != 0
@@ -780,9 +780,11 @@ def test_attn_prefill_float_aligned(pos0):
                                    (16384, 512, 40), (28672, 256, 64),
                                    # few tiles for the CUs: one ragged token tile over 27
                                    # K stages; 30 and 40 256x128 tiles' worth; 160 of them
-                                   # (5/8 of the CUs) with a ragged last token tile
+                                   # with a ragged last token tile
                                    (2560, 6912, 65), (2560, 2560, 300), (5120, 4096, 200),
-                                   (2560, 2560, 2000)])
+                                   (2560, 2560, 2000),
+                                   # 130 of them: 128x128 tiles instead, a few CUs with two
+                                   (2560, 512, 1640)])
 def test_gemm_mfma_bitexact(N, K, n):
     rng = np.random.default_rng(N + n)
     w = ternary(rng, N, K)
@@ -801,11 +803,14 @@ def test_gemm_mfma_bitexact(N, K, n):
 
 # Grids of more than one round over the CUs: 256x256 tiles for long rows (5 and
 # 6 token tiles, the last of 6 tokens or one; 14 of them over 10 feature
-# tiles), 128x128 tiles two per CU for short ones (one and ten K stages of 256,
-# ragged last tiles), and 128x128 where N is no multiple of 256.  Every epilogue,
-# on the rows at the tiles' edges and a few between
+# tiles) and for short ones whose second round is more than half full (7 over
+# 32), 128x128 tiles two per CU for short ones (one and ten K stages of 256,
+# ragged last tiles), and 128x128 where N is no multiple of 256.  The store,
+# residual and gate|up epilogues (q|k|v: below), on the rows at the tiles' edges
+# and a few between
 @pytest.mark.parametrize("N,K,n", [(8192, 4096, 1030), (8192, 4096, 1281), (2560, 6912, 3330),
-                                   (13824, 256, 600), (3840, 2560, 2300), (4224, 512, 1030)])
+                                   (13824, 256, 600), (3840, 2560, 2300), (4224, 512, 1030),
+                                   (8192, 512, 1700)])
 def test_gemm_large_grids_bitexact(N, K, n):
     rng = np.random.default_rng(N + K + n)
     Wn = synth.i2s_pack(ternary(rng, N, K))
