@@ -2672,13 +2672,14 @@ static int launch_prefill(const float *q, const uint16_t *kc, const uint16_t *vc
     return 0;
 }
 
-// pairs of queries for G >= 4 when both fit the LDS budget (smaller groups
-// keep one query per workgroup: their pair variants do not fit registers)
+// pairs of queries for G = 4 when both fit the LDS budget (smaller groups keep
+// one query per workgroup: their pair variants do not fit registers; a pair of
+// G = 8 fits only rows that run on MFMA)
 template <int G>
 static int launch_prefill_g(const float *q, const uint16_t *kc, const uint16_t *vc, int pos0,
                             int n_q, int H, int Hkv, int max_seq, int s_max, float *out,
                             hipStream_t s) {
-    if constexpr (G >= 4) {
+    if constexpr (G == 4) {
         if (prefill_smem(2 * G, s_max) <= kPrefillLds)
             return launch_prefill<G, 2>(q, kc, vc, pos0, n_q, H, Hkv, max_seq, s_max, out, s);
     }
