@@ -1194,9 +1194,10 @@ __global__ __launch_bounds__(kPrefillThreads) void attn_prefill_kernel(
 // B[k l/16][col l%16] and holds D[row 4(l/16) + i][col l%16] in register i.
 // One dependent chain issues at 32 cycles per instruction, the MFMA's own
 // rate; a VALU instruction between two of them costs it 8 to 16 cycles, also
-// when other waves wait (measured with chains in registers: no VALU 147
-// TFLOP/s from four waves per SIMD, one convert per MFMA 122, from one wave
-// 130 and 96), so the loops below hold MFMAs, loads and nothing else.
+// when other waves wait (measured with chains in registers over 0.7 ms: no VALU
+// 150 TFLOP/s from four waves per SIMD, one convert per MFMA 122, from one wave
+// 130 and 96; over longer runs 155), so the loops below hold MFMAs, loads and
+// nothing else.
 //
 // The A operands come from f32 copies of the cache laid out for them
 // (attn_kv_tiles_kernel, one pass per call), per KV head and 16 positions:
@@ -1333,7 +1334,8 @@ __global__ __launch_bounds__(256) void attn_kv_tiles_kernel(const uint16_t *__re
 // 4 apart (strides 128 .. 16), the components (8, 4), then lanes 2, 1 apart.
 // The row holds raw dots (scaled here, which makes them canonical, so the max
 // needs no extra instructions).  256 (NJ - 1) < S <= 256 NJ: only the last
-// group is masked.  In place; slots of positions >= S become zeros.
+// group is masked.  In place; within the NJ groups, slots of positions >= S
+// become zeros (later slots keep what they hold).
 template <int NJ>
 __device__ __forceinline__ void softmax_row_slots(float *row, float scale, int S, int Sw,
                                                   int lane) {
@@ -1470,6 +1472,7 @@ __global__ __launch_bounds__(kPfmThreads, R == 16 ? 4 : 2) void attn_prefill_mfm
     const int nb = len0 >> 4, last = nt - 1;   // whole batches; the last one
     const CopyRsrc vt = copy_rsrc(Vt, hk, ntile_ws);
     constexpr int NV = kPvAhead + 1;
+    static_assert(NV % 2 == 0, "p's two buffers keep their parity from pass to pass");
     float4 vr[NV], vtail[2];
     auto loadv = [&](float4 &v, int b) {
         __builtin_amdgcn_sched_barrier(0);
