@@ -570,12 +570,12 @@ def test_attn_decode_fused_rejects_unsupported():
                         np.zeros((4, 8, 128), np.float16), 3, 32, 4, 128, 8, fused=True)
 
 
-# Rows up to 2368 positions run on the f32-MFMA kernel (16 score rows per
-# workgroup: 16/G queries, so for G = 1 and 2 the four rows of one P.V chain
-# group have different lengths; ragged last blocks; (0, 257) pairs rows of 256
-# and 257 positions; rows shorter than a 16-position batch), longer ones on
-# the VALU kernel (G = 4 and 8 take query pairs, G = 1, 2 one query per
-# workgroup)
+# Rows up to 2496 positions run on the f32-MFMA kernel with 16 score rows per
+# workgroup (16/G queries, so for G = 1 and 2 the rows of one workgroup have
+# many lengths; ragged last blocks; (0, 257) pairs rows of 256 and 257
+# positions; rows shorter than a 16-position batch), rows up to 5056 with 8,
+# longer ones on the VALU kernel (one query per workgroup; G = 1, 2 and 4, rows
+# of a length that is and is not a multiple of 4 and of 16)
 @pytest.mark.parametrize("H,Hkv,S,pos0,n", [(20, 5, 256, 30, 100), (20, 5, 512, 0, 257),
                                             (16, 2, 1200, 900, 31), (8, 8, 300, 5, 40),
                                             (16, 8, 300, 100, 33), (20, 5, 2100, 2040, 9),
@@ -583,11 +583,13 @@ def test_attn_decode_fused_rejects_unsupported():
                                             (8, 4, 200, 13, 37), (4, 4, 300, 250, 11),
                                             # 1001 queries over 4 P.V blocks, a lone last query
                                             (20, 5, 1100, 50, 1001),
-                                            # the longest rows the MFMA kernel takes
                                             (20, 5, 2368, 2300, 68),
-                                            # VALU kernel: rows past 2368 positions
+                                            # 16 score rows, then 8 (rows of 2497 or more)
                                             (20, 5, 2600, 2369, 30), (16, 8, 3000, 2900, 17),
                                             (8, 8, 2500, 2450, 11),
+                                            # VALU kernel: rows past 5056 positions
+                                            (4, 4, 5070, 5054, 9), (4, 2, 5064, 5053, 11),
+                                            (8, 2, 5200, 5190, 10),
                                             # few queries of long rows with G = 1, 2: VALU at
                                             # rows of 2369 or more, MFMA where the K / V of an
                                             # XCD's workgroups pass 4 MB (4 of 2420, 5 of 3000)
@@ -607,7 +609,7 @@ def test_attn_prefill_causal_bitexact(H, Hkv, S, pos0, n):
     assert np.array_equal(out, ref)
 
 
-# Edges of the f32-MFMA prefill attention: its P.V runs 32 positions per batch,
+# Edges of the f32-MFMA prefill attention: its P.V runs 16 positions per batch,
 # then groups of four, then single steps where the rows' lengths differ, so
 # lengths sit on each side of 4, 16 and 32; rows past 2496 positions take 8
 # score rows per workgroup (up to 5056), longer ones the VALU kernel
@@ -629,6 +631,58 @@ def test_attn_prefill_length_edges(H, Hkv, pos0, n):
     ref = _oracle_attn(q.reshape(-1), kc, vc, n, S, H, Hkv, hd).reshape(n, H * hd)
     assert np.array_equal(out, ref, equal_nan=True)
     assert np.isfinite(out[:-1]).all()
+
+
+def _hard_values(kind, rng, n, H, Hkv, S, hd):
+    """q, K and V whose sums show any step that is not one fused multiply-add
+    in order, rounded to f32 with subnormals kept."""
+    def f16(m, lo, hi):   # random sign and mantissa, exponent uniform in [lo, hi)
+        e = rng.integers(lo, hi, m).astype(np.float64)
+        return (rng.choice([-1.0, 1.0], m) * (1 + rng.random(m)) * 2.0 ** e).astype(np.float16)
+
+    kv = (Hkv, S, hd)
+    q = rng.standard_normal((n, H, hd))
+    k, v = rng.standard_normal(kv) * 0.7, f16(kv, -24, 15)
+    if kind == "tails":
+        # half of the positions score about 95 below the others: subnormal
+        # probabilities, alone in the dims where the others' V is 0
+        u, far = rng.choice([-1.0, 1.0], hd), rng.random(S) < 0.5
+        q = 8 * u + 0.5 * q
+        k = np.where(far[:, None], -1.05 * u, 0.0) + 0.02 * rng.standard_normal(kv)
+        v[..., 0::2] *= far[:, None]
+    elif kind == "subnormal":     # K of f16 subnormals only
+        q *= 2.0 ** 17
+        k = f16(kv, -24, -14)
+    elif kind == "cancel":        # terms of +-7000 cancel to scores of about 4
+        base = rng.uniform(20.0, 30.0, (*kv[:2], hd // 4)) * 1000
+        k = np.repeat(base, 4, -1) * np.tile([1.0, -1.0, -1.0, 1.0], hd // 4)
+        k = k + rng.standard_normal(kv) * 16
+        q = np.repeat(rng.standard_normal((n, H, hd // 4)) * 0.25, 4, -1)
+        v = rng.choice([-1.0, 1.0], kv) * rng.uniform(6e4, 6.5e4, kv)
+    elif kind == "wide":          # score terms over 60 binary orders
+        q = q * 2.0 ** rng.integers(-40, 6, q.shape)
+        k = f16(kv, -14, 2)
+    elif kind == "overflow":      # sums past the largest f32 before terms that would bring them back
+        q = np.tile([2.0, 2.0, -2.0, -2.0], hd // 4) * np.ones_like(q) * 1e38 \
+            * (rng.random((n, H, 1)) < 0.3) + q
+        k = np.ones(kv) + (rng.random((*kv[:2], 1)) < 0.2) * rng.standard_normal(kv)
+    else:
+        raise ValueError(kind)
+    return (q.reshape(n, H * hd).astype(np.float32), np.asarray(k).astype(np.float16),
+            np.asarray(v).astype(np.float16))
+
+
+# The prefill attention adds four products per instruction: values that would
+# show products added in another order or in a wider sum, or subnormals
+# flushed, with 16 and with 8 score rows per workgroup
+@pytest.mark.parametrize("kind", ["tails", "subnormal", "cancel", "wide", "overflow"])
+@pytest.mark.parametrize("H,Hkv,pos0,n", [(20, 5, 301, 21), (8, 8, 40, 37), (20, 5, 2600, 5)])
+def test_attn_prefill_hard_values_bitexact(kind, H, Hkv, pos0, n):
+    hd, S = 128, pos0 + n
+    q, kc, vc = _hard_values(kind, np.random.default_rng([pos0, n]), n, H, Hkv, S, hd)
+    out = ops.attn_prefill(q, kc, vc, n, pos0, H, Hkv, hd, S)
+    ref = _oracle_attn(q.reshape(-1), kc, vc, n, S, H, Hkv, hd).reshape(n, H * hd)
+    assert np.array_equal(out, ref, equal_nan=True)
 
 
 # A captured call past 2368 positions allocates nothing (VALU kernel: query
@@ -829,6 +883,51 @@ def test_gemm_large_grids_bitexact(N, K, n):
         acc, Y, _ = ops.gemm(Wt, x, g, 1e-5, ws, N, K, epilogue=epi, Y0=r if epi == 1 else None)
         assert np.array_equal(acc[rows], acc_o), epi
         assert np.array_equal(Y[rows], want[epi]), epi
+
+
+# The q|k|v epilogue (RoPE, K / V append) on the same tiles: 128x128 at the 2B
+# projection's width, 256x256 for long rows, both with a ragged last token tile
+# behind cached positions, and one round of 256x128.  Rows past the new ones
+# stay as they were.
+@pytest.mark.parametrize("H,Hkv,K,n,pos0", [(20, 5, 2560, 2300, 37), (32, 8, 4096, 1400, 5),
+                                            (20, 5, 512, 1500, 3)])
+def test_gemm_qkv_large_grids_bitexact(H, Hkv, K, n, pos0):
+    hd, theta = 128, 500000.0
+    Dq, Dkv, max_seq = H * hd, Hkv * hd, pos0 + n + 3
+    N = Dq + 2 * Dkv
+    rng = np.random.default_rng(N + K)
+    Wn = synth.i2s_pack(ternary(rng, N, K))
+    x = rng.standard_normal((n, K)).astype(np.float32)
+    g = rng.uniform(0.5, 1.5, K).astype(np.float32)
+    ws = rng.uniform(0.01, 0.02, N).astype(np.float32)
+    rows = sorted({t for b in range(0, n + 1, 128) for t in (b - 1, b) if 0 <= t < n} | {n - 1} |
+                  set(rng.integers(0, n, 8).tolist()))
+    xq, s = O.quantize(O.rmsnorm(x[rows], g, 1e-5))
+    _, Y = O.gemm(Wn, xq, ws, s, K)
+    rot = lambda a, heads: np.stack([O.rope(a[i], 1, heads, hd, pos0 + t, theta).reshape(-1)
+                                     for i, t in enumerate(rows)])
+    L = ops.lib()
+    Wt = ops.upload_ternary(Wn, K)
+    npad = (n + 63) // 64 * 64
+    dx, dg, dws = (ops.DeviceArray.from_host(a) for a in (x, g, ws))
+    Xt = ops.DeviceArray((npad * K,), np.int8, zero=True)
+    sc, sm = ops.DeviceArray((npad,), np.float32), ops.DeviceArray((npad,), np.int32)
+    ops.quantize_rows_tiled(dx, dg, 1e-5, n, K, Xt, sc, sm)
+    q = ops.DeviceArray((n, Dq), np.float32)
+    stale = np.full((Hkv, max_seq, hd), 0.25, np.float16)
+    kc, vc = (ops.DeviceArray.from_host(stale.view(np.uint16)) for _ in range(2))
+    rope = ops.DeviceArray.from_host(rope_table(max_seq, hd, theta))
+    ops.check(L.oxb_gemm_qkv(Wt.ptr, Xt.ptr, sc.ptr, sm.ptr, dws.ptr, Dq, Dkv, hd, K, n, pos0,
+                             q.ptr, kc.ptr, vc.ptr, max_seq, rope.ptr, None), "gemm_qkv")
+    ops.sync()
+    assert np.array_equal(q.download()[rows], rot(Y[:, :Dq], H))
+    at = [pos0 + t for t in rows]
+    for cache, want in ((kc, rot(Y[:, Dq:Dq + Dkv], Hkv)), (vc, Y[:, Dq + Dkv:])):
+        c = cache.download().view(np.float16)
+        new = want.reshape(-1, Hkv, hd).transpose(1, 0, 2).astype(np.float16)
+        assert np.array_equal(c[:, at], new)
+        assert np.array_equal(c[:, :pos0], stale[:, :pos0])
+        assert np.array_equal(c[:, pos0 + n:], stale[:, pos0 + n:])
 
 
 # the split GEMMs' arrival counters: a fixed area at the start of a workspace

@@ -627,6 +627,16 @@ def test_batch_rejects_unprefilled_slot():
     m.close()
 
 
+def test_long_prompt_on_two_round_gemm_grids():
+    """A 2300-token prompt at the 2B model's attention width (one layer): its
+    q|k|v GEMM needs more than one round over the CUs and writes the octet copy
+    of V that the decode steps after it read."""
+    cfg = synth.small_config(n_layers=1, hidden=2560, heads=20, kv_heads=5, context=4096)
+    path = synth.cached_gguf(cfg, seed=32)
+    prompt = np.random.default_rng(32).integers(0, cfg.vocab, 2300).astype(np.int32)
+    _greedy_parity(path, prompt, 4)
+
+
 def test_prefill_workspace_follows_the_context():
     """The prefill attention's workspace is sized by the model's context (4 KV
     heads: 20 MB for the longest rows the kernel takes, 256 KB for 64), and a
